@@ -58,10 +58,33 @@ int fail(const char *fmt, ...)
 
 // ------------------------------------------------------------------ params
 
+// t / d for 0 <= t < 2^31 by a multiplication: the update kernels find a tile's
+// row and column with it before their first load (a plain division took 35
+// instructions there)
+struct FastDiv {
+    unsigned m;     // ceil(2^(31 + s) / d), s = ceil(log2(d))
+    int s;
+    int d;
+};
+inline FastDiv fast_div(int d)
+{
+    FastDiv f{ 0, 0, d };
+    while ((1ll << f.s) < d) ++f.s;
+    f.m = (unsigned)(((1ull << (31 + f.s)) + (unsigned)d - 1) / (unsigned)d);
+    return f;
+}
+__host__ __device__ __forceinline__ int div_by(const FastDiv &f, int t)
+{
+    return (int)(((unsigned long long)(unsigned)t * f.m) >> (31 + f.s));
+}
+
 struct Grid {
     int nx, ny, pitch, fw, abs_type, free_surf, weq, L, nd;
     int gx2, gx3, gy2, gy3;
     int plane;      // floats per padded plane
+    FastDiv tdiv[3];    // division by the tiles per row of the shapes of 1, 2 and 4 cells per thread
+    // tile rows of the lower absorbing frame, in tiles of BY and of VROWS BY rows
+    struct { int first, n; } low[2];
     int wx, wy;     // row lengths of x-frame and y-frame CPML memory
     int ntx;        // tiles along x of the one-cell-per-thread update kernels
     int nty;        // tiles along y of the same
@@ -142,6 +165,8 @@ struct Fields {
     }
 };
 
+using float4v = float __attribute__((ext_vector_type(4)));
+
 struct Mat {
     const float *rip, *rjp;
     const float *f, *g, *fipjp;                 // EL_ISO / VEL_ISO
@@ -153,6 +178,9 @@ struct Mat {
     const float *pu, *ppi, *ptaus, *ptaup;      // snapshots
     const float *surf;                          // free-surface coefficients of row 1, SURF_N x NX
     const float *prof;                          // CPML profiles, 12 x (2FW+1)
+    // b, a, b at half points, a at half points of frame index h (2FW+1 each)
+    const float4v *pmlx, *pmly;
+    int kone;                                   // every K of the profiles is 1 (K_MAX_CPML = 1)
     float eta[SOFI_MAXL + 1], bip[SOFI_MAXL + 1], cip[SOFI_MAXL + 1];
     float bjm[SOFI_MAXL + 1];                   // free surface: eta_l / (1 + eta_l / 2)
 };
@@ -212,30 +240,114 @@ __device__ __forceinline__ void op_s(const Grid &g, const float *__restrict__ vx
     vyy = e * g.dhi;
 }
 
+// What CPML adds to a frame cell's update, its memory and the x profiles, is
+// fetched straight into LDS when the update's stencils are, and read from
+// there once these are done, so that no register holds it meanwhile.  What
+// bounds small grids and the last tiles of large ones is the chain of trips to
+// memory of a frame wave: loaded where they are used, behind the frame's
+// branches, these values cost it up to four more.  With the fetch, same bits,
+// us per step before and after: EL_ISO FD4 400 x 400 13.3 and 10.2, EL_ISO FD8
+// 1500 x 500 23.9 and 20.1, 2000 x 1000 46.4 and 38.7, VEL_ISO L = 3 FD8 4000
+// x 2000 217 and 213.  Early loads into registers gave the small grids as much
+// but took 12 to 28 registers from every wave: 2 to 11 % off the interior.
+// Damping factors (ABS_TYPE 2) stay with their use: fetched early they gained
+// nothing.
+struct Park {                                   // of a wave's cells, one per lane
+    float4v cx[64];                             // b, a, b at half points, a at half points
+    float x0[64], x1[64], y0[64], y1[64];       // memory of sxx_x, sxy_x, syy_y, sxy_y or vxx, vyx, vyy, vxy
+};
+// A block's parks are its dynamic LDS, park_bytes() of them: none without CPML
+__device__ __forceinline__ Park *parks()
+{
+    extern __shared__ float4v park_lds[];
+    return reinterpret_cast<Park *>(park_lds);
+}
+
+struct Frame {
+    bool xf, yf;                                // cell of the x / y frame
+    const Park *pk;
+    __device__ __forceinline__ bool any() const { return xf || yf; }
+};
+
+// 4 or 16 bytes per lane from src to LDS (dst: the wave's lane 0)
+__device__ __forceinline__ void to_lds(const float *src, float *dst)
+{
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
+                                     (__attribute__((address_space(3))) void *)dst, 4, 0, 0);
+}
+__device__ __forceinline__ void to_lds(const float4v *src, float4v *dst)
+{
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
+                                     (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
+}
+
+// V: for the velocity update, else the stress update; one wave per tile row
+// (j is the same in all its lanes), lane = threadIdx.x
+template <bool V>
+__device__ __forceinline__ Frame frame_load(const Grid &g, const Fields &f, const Mat &m, int i, int j, int c, Park &pk)
+{
+    const int ju = __builtin_amdgcn_readfirstlane(j);
+    Frame o;
+    o.xf = in_xframe(g, i);
+    o.yf = in_yframe(g, ju);
+    o.pk = &pk;
+    if (g.abs_type == 1) {
+        if (o.yf) {
+            const int q = hy(g, ju) * g.wy + i;
+            to_lds((V ? f.psi_syy_y : f.psi_vyy) + q, pk.y0);
+            to_lds((V ? f.psi_sxy_y : f.psi_vxy) + q, pk.y1);
+        }
+        if (o.xf) {
+            const int h = hx(g, i), q = ju * g.wx + h;
+            to_lds(m.pmlx + h, pk.cx);
+            to_lds((V ? f.psi_sxx_x : f.psi_vxx) + q, pk.x0);
+            to_lds((V ? f.psi_sxy_x : f.psi_vyx) + q, pk.x1);
+        }
+    }
+    return o;
+}
+
+// the fetches to LDS have arrived (vmcnt 0)
+__device__ __forceinline__ void frame_wait()
+{
+    __builtin_amdgcn_s_waitcnt(0x0f70);
+    asm volatile("" ::: "memory");
+}
+
+// x / K of profile k at h
+__device__ __forceinline__ float div_k(const Grid &g, const Mat &m, float x, int k, int h)
+{
+    return m.kone ? x : x / PRF(g, m, k, h);
+}
+
 // CPML on the stress-side derivatives of one frame cell (cpml_update_s_x/_y,
 // src/cpml_update.c:30-46); updates the psi memory and returns modified values.
-__device__ __forceinline__ void cpml_dv(const Grid &g, const Mat &m, Fields &f, int i, int j, bool xf, bool yf,
+__device__ __forceinline__ void cpml_dv(const Grid &g, const Mat &m, Fields &f, const Frame &o, int i, int j,
                                         float &vxx, float &vyx, float &vxy, float &vyy)
 {
-    if (xf) {
+    const int lane = threadIdx.x;
+    frame_wait();
+    if (o.xf) {
         const int h = hx(g, i);
-        const int o = j * g.wx + h;
-        float px = PRF(g, m, SOFI_P_B_X, h) * f.psi_vxx[o] + PRF(g, m, SOFI_P_A_X, h) * vxx;
-        f.psi_vxx[o] = px;
-        vxx = vxx / PRF(g, m, SOFI_P_K_X, h) + px;
-        float py = PRF(g, m, SOFI_P_B_X_HALF, h) * f.psi_vyx[o] + PRF(g, m, SOFI_P_A_X_HALF, h) * vyx;
-        f.psi_vyx[o] = py;
-        vyx = vyx / PRF(g, m, SOFI_P_K_X_HALF, h) + py;
+        const int q = j * g.wx + h;
+        const auto cx = o.pk->cx[lane];
+        const float px = __builtin_fmaf(cx[0], o.pk->x0[lane], cx[1] * vxx);
+        f.psi_vxx[q] = px;
+        vxx = div_k(g, m, vxx, SOFI_P_K_X, h) + px;
+        const float py = __builtin_fmaf(cx[2], o.pk->x1[lane], cx[3] * vyx);
+        f.psi_vyx[q] = py;
+        vyx = div_k(g, m, vyx, SOFI_P_K_X_HALF, h) + py;
     }
-    if (yf) {
-        const int h = hy(g, j);
-        const int o = h * g.wy + i;
-        float py = PRF(g, m, SOFI_P_B_Y, h) * f.psi_vyy[o] + PRF(g, m, SOFI_P_A_Y, h) * vyy;
-        f.psi_vyy[o] = py;
-        vyy = vyy / PRF(g, m, SOFI_P_K_Y, h) + py;
-        float px = PRF(g, m, SOFI_P_B_Y_HALF, h) * f.psi_vxy[o] + PRF(g, m, SOFI_P_A_Y_HALF, h) * vxy;
-        f.psi_vxy[o] = px;
-        vxy = vxy / PRF(g, m, SOFI_P_K_Y_HALF, h) + px;
+    if (o.yf) {
+        const int h = hy(g, __builtin_amdgcn_readfirstlane(j));
+        const int q = h * g.wy + i;
+        const auto cy = m.pmly[h];
+        const float py = __builtin_fmaf(cy[0], o.pk->y0[lane], cy[1] * vyy);
+        f.psi_vyy[q] = py;
+        vyy = div_k(g, m, vyy, SOFI_P_K_Y, h) + py;
+        const float px = __builtin_fmaf(cy[2], o.pk->y1[lane], cy[3] * vxy);
+        f.psi_vxy[q] = px;
+        vxy = div_k(g, m, vxy, SOFI_P_K_Y_HALF, h) + px;
     }
 }
 
@@ -528,7 +640,16 @@ __global__ void k_surface(Grid g, Fields f0, Mat m)
 // fetched it).  Measured on the 4000 x 2000 viscoelastic workload, this
 // order beat giving each XCD a contiguous band of its own by 4 % (stress)
 // and 3 % (velocity).
-__device__ __forceinline__ int tile_id() { return blockIdx.x; }
+// The tile rows of the lower absorbing frame come first: their tiles take
+// longer than the others, and a launch that ends with them ends late (EL_ISO
+// FD8 with CPML, us per step with and without: 1500 x 500 20.1 and 21.1, 2000 x
+// 1000 38.8 and 39.1, 2741 x 1313 59.2 and 59.7).
+// Block b's tile: 2^vw cells per thread in x, rows in y as of g.low[k].
+__device__ __forceinline__ int2 tile_of(const Grid &g, int k, int vw, int b)
+{
+    const int r = div_by(g.tdiv[vw], b), n = g.low[k].n;
+    return make_int2(b - r * g.tdiv[vw].d, r < n ? g.low[k].first + r : r - n);
+}
 
 // Tile shapes: CELL, one thread per cell in BX x BY tiles (also the TTI
 // passes); VEC2 / VEC4, one thread per VW = 2 / 4 consecutive cells of a row
@@ -598,36 +719,40 @@ __device__ __forceinline__ void stv(float *p, int c, vecf<VW> v)
 // derivatives of op_v (no 1/DH), on the cell's velocities in registers.
 // cpml_update_v_x / _y (src/cpml_update.c:50-66) on the stress derivatives of
 // a frame cell
-__device__ __forceinline__ void cpml_v(const Grid &g, Fields &f, const Mat &m, int i, int j, bool xf, bool yf,
+__device__ __forceinline__ void cpml_v(const Grid &g, Fields &f, const Mat &m, const Frame &o, int i, int j,
                                        float &sxx_x, float &sxy_x, float &sxy_y, float &syy_y)
 {
-    if (xf) {
-        const int h = hx(g, i), o = j * g.wx + h;
-        float a = PRF(g, m, SOFI_P_B_X_HALF, h) * f.psi_sxx_x[o] + PRF(g, m, SOFI_P_A_X_HALF, h) * sxx_x;
-        f.psi_sxx_x[o] = a;
-        sxx_x = sxx_x / PRF(g, m, SOFI_P_K_X_HALF, h) + a;
-        float b = PRF(g, m, SOFI_P_B_X, h) * f.psi_sxy_x[o] + PRF(g, m, SOFI_P_A_X, h) * sxy_x;
-        f.psi_sxy_x[o] = b;
-        sxy_x = sxy_x / PRF(g, m, SOFI_P_K_X, h) + b;
+    const int lane = threadIdx.x;
+    frame_wait();
+    if (o.xf) {
+        const int h = hx(g, i), q = j * g.wx + h;
+        const auto cx = o.pk->cx[lane];
+        const float a = __builtin_fmaf(cx[2], o.pk->x0[lane], cx[3] * sxx_x);
+        f.psi_sxx_x[q] = a;
+        sxx_x = div_k(g, m, sxx_x, SOFI_P_K_X_HALF, h) + a;
+        const float b = __builtin_fmaf(cx[0], o.pk->x1[lane], cx[1] * sxy_x);
+        f.psi_sxy_x[q] = b;
+        sxy_x = div_k(g, m, sxy_x, SOFI_P_K_X, h) + b;
     }
-    if (yf) {
-        const int h = hy(g, j), o = h * g.wy + i;
-        float a = PRF(g, m, SOFI_P_B_Y_HALF, h) * f.psi_syy_y[o] + PRF(g, m, SOFI_P_A_Y_HALF, h) * syy_y;
-        f.psi_syy_y[o] = a;
-        syy_y = syy_y / PRF(g, m, SOFI_P_K_Y_HALF, h) + a;
-        float b = PRF(g, m, SOFI_P_B_Y, h) * f.psi_sxy_y[o] + PRF(g, m, SOFI_P_A_Y, h) * sxy_y;
-        f.psi_sxy_y[o] = b;
-        sxy_y = sxy_y / PRF(g, m, SOFI_P_K_Y, h) + b;
+    if (o.yf) {
+        const int h = hy(g, __builtin_amdgcn_readfirstlane(j)), q = h * g.wy + i;
+        const auto cy = m.pmly[h];
+        const float a = __builtin_fmaf(cy[2], o.pk->y0[lane], cy[3] * syy_y);
+        f.psi_syy_y[q] = a;
+        syy_y = div_k(g, m, syy_y, SOFI_P_K_Y_HALF, h) + a;
+        const float b = __builtin_fmaf(cy[0], o.pk->y1[lane], cy[1] * sxy_y);
+        f.psi_sxy_y[q] = b;
+        sxy_y = div_k(g, m, sxy_y, SOFI_P_K_Y, h) + b;
     }
 }
 
 __device__ __forceinline__ void velocity_core(const Grid &g, Fields &f, const Mat &m, const Src &s, const Fuse &fz,
-                                              int nt, int i, int j, int c, float sxx_x, float sxy_x, float sxy_y,
+                                              const Frame &fr, int nt, int i, int j, int c, float sxx_x, float sxy_x, float sxy_y,
                                               float syy_y, float rip, float rjp, float &vx, float &vy)
 {
     // instability guard of time_loop (src/time_loop.c:44-47), before this step's update
     if (i == g.nx / 2 && j == g.ny / 2 && isnan(vy) && *f.unstable == 0) *f.unstable = step_of(fz.ntb, nt);
-    const bool xf = in_xframe(g, i), yf = in_yframe(g, j), frame = xf || yf;
+    const bool frame = fr.any();
     if (frame && g.abs_type != 1 && g.abs_type != 2) {
         // a frame that is never updated still receives its forces (the
         // reference adds them to every source cell first)
@@ -635,7 +760,7 @@ __device__ __forceinline__ void velocity_core(const Grid &g, Fields &f, const Ma
             if (c == fz.c[k]) force_add(g, s, fz.soff + k, step_of(fz.ntb, nt), rip, rjp, vx, vy);
         return;
     }
-    if (g.abs_type == 1 && frame) cpml_v(g, f, m, i, j, xf, yf, sxx_x, sxy_x, sxy_y, syy_y);
+    if (g.abs_type == 1 && frame) cpml_v(g, f, m, fr, i, j, sxx_x, sxy_x, sxy_y, syy_y);
     for (int k = 0; k < fz.nforce; ++k)
         if (c == fz.c[k]) force_add(g, s, fz.soff + k, step_of(fz.ntb, nt), rip, rjp, vx, vy);
     if (fz.fwi_acc == 1) {
@@ -677,9 +802,10 @@ __device__ __forceinline__ void velocity_core(const Grid &g, Fields &f, const Ma
 // tile t of BX x TBY cells (tiles row by row, g.ntx to a row)
 template <int ND, bool ONE, bool NT, int TBY = BY>
 __device__ __forceinline__ void velocity_tile(const Grid &g, const Fields &f0, const Mat &m, const Src &s,
-                                              const Fuse &fz, int nt, int t)
+                                              const Fuse &fz, int nt, int tx, int ty)
 {
-    const int ty = t / g.ntx, tx = t - ty * g.ntx;
+    Park *const park = parks();
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
     const int i = 1 + tx * BX + threadIdx.x;
     const int j = 1 + ty * TBY + threadIdx.y;
     if (i > g.nx || j > g.ny) return;
@@ -688,10 +814,11 @@ __device__ __forceinline__ void velocity_tile(const Grid &g, const Fields &f0, c
     const int k0 = ONE ? 0 : g.k_lo + blockIdx.y * g.spt, k1 = ONE ? 1 : min(k0 + g.spt, g.k_hi);
     for (int k = k0; k < k1; ++k) {
         Fields f = ONE ? f0 : f0.at(k, g);
+        const Frame fr = frame_load<true>(g, f, m, i, j, c, park[w]);
         float sxx_x, sxy_x, sxy_y, syy_y;
         op_v<ND>(g, f.sxx, f.syy, f.sxy, c, sxx_x, sxy_x, sxy_y, syy_y);
         float vx = ld1<NT>(f.vx, c), vy = ld1<NT>(f.vy, c);
-        velocity_core(g, f, m, s, fz, nt, i, j, c, sxx_x, sxy_x, sxy_y, syy_y, rip, rjp, vx, vy);
+        velocity_core(g, f, m, s, fz, fr, nt, i, j, c, sxx_x, sxy_x, sxy_y, syy_y, rip, rjp, vx, vy);
         st1<NT>(f.vx, c, vx);
         st1<NT>(f.vy, c, vy);
     }
@@ -699,7 +826,8 @@ __device__ __forceinline__ void velocity_tile(const Grid &g, const Fields &f0, c
 template <int ND, bool ONE, bool NT = ONE>
 __global__ __launch_bounds__(BX *BY) void k_velocity(Grid g, Fields f0, Mat m, Src s, Fuse fz, int nt)
 {
-    velocity_tile<ND, ONE, NT>(g, f0, m, s, fz, nt, tile_id());
+    const int2 t = tile_of(g, 0, 0, blockIdx.x);
+    velocity_tile<ND, ONE, NT>(g, f0, m, s, fz, nt, t.x, t.y);
 }
 
 // The one-shot velocity update (one slot, one thread per cell) with R
@@ -715,12 +843,20 @@ constexpr int VROWS = 2;
 template <int ND, bool NT, int R>
 __global__ __launch_bounds__(BX *BY) void k_velocity_r(Grid g, Fields f, Mat m, Src s, Fuse fz, int nt)
 {
-    const int t = tile_id(), ty = t / g.ntx, tx = t - ty * g.ntx;
+    Park(*const park)[R] = reinterpret_cast<Park(*)[R]>(parks());
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int2 t = tile_of(g, 1, 0, blockIdx.x);
+    const int tx = t.x, ty = t.y;
     const int i = 1 + tx * BX + threadIdx.x;
+    static_assert(R == VROWS, "tile_of's rows");
     const int j = 1 + ty * R * BY + R * threadIdx.y;
     if (i > g.nx || j > g.ny) return;
     const int nr = min(R, g.ny - j + 1);
     const int c = IDX(g, i, j), P = g.pitch;
+    Frame fr[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+        if (q < nr) fr[q] = frame_load<true>(g, f, m, i, j + q, c + q * P, park[w][q]);
     // rows j - ND .. j + ND + R - 2 of sxy and j - ND + 1 .. j + ND + R - 1 of syy
     float qy[2 * ND + R - 1], qs[2 * ND + R - 1];
 #pragma unroll
@@ -744,7 +880,7 @@ __global__ __launch_bounds__(BX *BY) void k_velocity_r(Grid g, Fields f, Mat m, 
         }
         const float rip = ld1<NT>(m.rip, cq), rjp = ld1<NT>(m.rjp, cq);
         float vx = ld1<NT>(f.vx, cq), vy = ld1<NT>(f.vy, cq);
-        velocity_core(g, f, m, s, fz, nt, i, j + q, cq, a, b, d, e, rip, rjp, vx, vy);
+        velocity_core(g, f, m, s, fz, fr[q], nt, i, j + q, cq, a, b, d, e, rip, rjp, vx, vy);
         st1<NT>(f.vx, cq, vx);
         st1<NT>(f.vy, cq, vy);
     }
@@ -755,7 +891,7 @@ __global__ __launch_bounds__(BX *BY) void k_velocity_r(Grid g, Fields f, Mat m, 
 // padding values
 template <int ND, int VW, bool PRE>
 __device__ __forceinline__ void velocity_v_slot(const Grid &g, Fields f, const Mat &m, const Src &s, const Fuse &fz,
-                                                int nt, int i0, int j, const vecf<VW> *pre)
+                                                int nt, int i0, int j, const vecf<VW> *pre, Park *park)
 {
     constexpr int G = (ND + VW - 1) / VW;
     using V = vecf<VW>;
@@ -770,28 +906,30 @@ __device__ __forceinline__ void velocity_v_slot(const Grid &g, Fields f, const M
             xy[(q + G) * VW + k] = b[k];
         }
     }
+    // sxy rows j + m - 1 and j - m, syy rows j + m and j - m + 1
+    V a1[ND], a0[ND], b1[ND], b0[ND];
+#pragma unroll
+    for (int mm = 1; mm <= ND; ++mm) {
+        if (mm > 1) a1[mm - 1] = ldv<VW>(f.sxy, c0 + (mm - 1) * P);
+        a0[mm - 1] = ldv<VW>(f.sxy, c0 - mm * P);
+        b1[mm - 1] = ldv<VW>(f.syy, c0 + mm * P);
+        b0[mm - 1] = ldv<VW>(f.syy, c0 - (mm - 1) * P);
+    }
+    V vx = ldv<VW>(f.vx, c0), vy = ldv<VW>(f.vy, c0);
+    const V rip = PRE ? pre[0] : ldv<VW>(m.rip, c0), rjp = PRE ? pre[1] : ldv<VW>(m.rjp, c0);
+    Frame fr[VW];      // (a cell past NX fetches the neighbouring entries, which nothing uses)
+#pragma unroll
+    for (int k = 0; k < VW; ++k) fr[k] = frame_load<true>(g, f, m, i0 + k, j, c0 + k, park[k]);
     float d[VW] = {}, e[VW] = {};
 #pragma unroll
     for (int mm = 1; mm <= ND; ++mm) {
         const float h = g.hc[mm];
-        // sxy rows j + m - 1 and j - m, syy rows j + m and j - m + 1
-        V a1;
-        if (mm == 1) {
-#pragma unroll
-            for (int k = 0; k < VW; ++k) a1[k] = xy[G * VW + k];
-        } else {
-            a1 = ldv<VW>(f.sxy, c0 + (mm - 1) * P);
-        }
-        const V a0 = ldv<VW>(f.sxy, c0 - mm * P);
-        const V b1 = ldv<VW>(f.syy, c0 + mm * P), b0 = ldv<VW>(f.syy, c0 - (mm - 1) * P);
 #pragma unroll
         for (int k = 0; k < VW; ++k) {
-            d[k] += h * (a1[k] - a0[k]);
-            e[k] += h * (b1[k] - b0[k]);
+            d[k] += h * ((mm == 1 ? xy[G * VW + k] : a1[mm - 1][k]) - a0[mm - 1][k]);
+            e[k] += h * (b1[mm - 1][k] - b0[mm - 1][k]);
         }
     }
-    V vx = ldv<VW>(f.vx, c0), vy = ldv<VW>(f.vy, c0);
-    const V rip = PRE ? pre[0] : ldv<VW>(m.rip, c0), rjp = PRE ? pre[1] : ldv<VW>(m.rjp, c0);
 #pragma unroll
     for (int k = 0; k < VW; ++k) {
         if (i0 + k > g.nx) break;
@@ -803,7 +941,7 @@ __device__ __forceinline__ void velocity_v_slot(const Grid &g, Fields f, const M
             b += h * (xy[G * VW + k + mm - 1] - xy[G * VW + k - mm]);
         }
         float x = vx[k], y = vy[k];
-        velocity_core(g, f, m, s, fz, nt, i0 + k, j, c0 + k, a, b, d[k], e[k], rip[k], rjp[k], x, y);
+        velocity_core(g, f, m, s, fz, fr[k], nt, i0 + k, j, c0 + k, a, b, d[k], e[k], rip[k], rjp[k], x, y);
         vx[k] = x;
         vy[k] = y;
     }
@@ -815,20 +953,22 @@ __device__ __forceinline__ void velocity_v_slot(const Grid &g, Fields f, const M
 template <int ND, int VW, bool ONE>
 __global__ __launch_bounds__(BX *BY) void k_velocity_v(Grid g, Fields f0, Mat m, Src s, Fuse fz, int nt)
 {
-    const int ntxv = (g.nx + BX * VW - 1) / (BX * VW);
-    const int t = tile_id(), ty = t / ntxv, tx = t - ty * ntxv;
+    Park(*const park)[VW] = reinterpret_cast<Park(*)[VW]>(parks());
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int2 t = tile_of(g, 0, VW / 2, blockIdx.x);
+    const int tx = t.x, ty = t.y;
     const int i0 = 1 + (tx * BX + threadIdx.x) * VW;
     const int j = 1 + ty * BY + threadIdx.y;
     if (i0 > g.nx || j > g.ny) return;
     if (ONE) {
-        velocity_v_slot<ND, VW, false>(g, f0, m, s, fz, nt, i0, j, nullptr);
+        velocity_v_slot<ND, VW, false>(g, f0, m, s, fz, nt, i0, j, nullptr, park[w]);
         return;
     }
     // a batch: the cells' coefficients once for the thread's slots
     const int c0 = IDX(g, i0, j);
     const vecf<VW> pre[2] = { ldv<VW>(m.rip, c0), ldv<VW>(m.rjp, c0) };
     const int k0 = g.k_lo + blockIdx.y * g.spt, k1 = min(k0 + g.spt, g.k_hi);
-    for (int k = k0; k < k1; ++k) velocity_v_slot<ND, VW, true>(g, f0.at(k, g), m, s, fz, nt, i0, j, pre);
+    for (int k = k0; k < k1; ++k) velocity_v_slot<ND, VW, true>(g, f0.at(k, g), m, s, fz, nt, i0, j, pre, park[w]);
 }
 
 // --------------------------------------------------------- stress updates
@@ -951,16 +1091,17 @@ __device__ __forceinline__ void visc_vti_final(float dthalbe, float u11, float u
 // Derivatives of a cell from the raw op_s sums (no 1/DH): scaled, and CPML in
 // the frame (cpml_update_s_x/_y).  Returns false for a frame cell that the
 // reference never updates (ABS_TYPE other than 1 or 2).
-__device__ __forceinline__ bool stress_dv(const Grid &g, Fields &f, const Mat &m, int i, int j, float a, float b,
-                                          float d, float e, float &vxx, float &vyx, float &vxy, float &vyy)
+__device__ __forceinline__ bool stress_dv(const Grid &g, Fields &f, const Mat &m, const Frame &fr, int i, int j,
+                                          float a, float b, float d, float e, float &vxx, float &vyx, float &vxy,
+                                          float &vyy)
 {
-    const bool xf = in_xframe(g, i), yf = in_yframe(g, j), frame = xf || yf;
+    const bool frame = fr.any();
     if (frame && g.abs_type != 1 && g.abs_type != 2) return false;
     vxx = a * g.dhi;
     vyx = b * g.dhi;
     vxy = d * g.dhi;
     vyy = e * g.dhi;
-    if (g.abs_type == 1 && frame) cpml_dv(g, m, f, i, j, xf, yf, vxx, vyx, vxy, vyy);
+    if (g.abs_type == 1 && frame) cpml_dv(g, m, f, fr, i, j, vxx, vyx, vxy, vyy);
     return true;
 }
 
@@ -971,9 +1112,9 @@ __device__ __forceinline__ bool stress_dv(const Grid &g, Fields &f, const Mat &m
 // correction of row 1).
 template <int ND, bool VISCO>
 __device__ __forceinline__ void stress_post(const Grid &g, Fields &f, const Mat &m, const Src &s, const Fuse &fz,
-                                            int nt, int i, int j, int c, float &sxx, float &syy, float &sxy)
+                                            const Frame &fr, int nt, int i, int j, int c, float &sxx, float &syy, float &sxy)
 {
-    if (g.abs_type == 2 && (in_xframe(g, i) || in_yframe(g, j))) {
+    if (g.abs_type == 2 && fr.any()) {
         const float q = m.absorb[c];
         sxy *= q;
         syy *= q;
@@ -1003,10 +1144,11 @@ __device__ __forceinline__ void stress_post(const Grid &g, Fields &f, const Mat 
 // slot, as in k_velocity).
 template <int ND, int WEQ, bool ONE, int TBY = BY>
 __device__ __forceinline__ void stress_tile(const Grid &g, const Fields &f0, const Mat &m, const Src &s,
-                                            const Fuse &fz, int nt, int t)
+                                            const Fuse &fz, int nt, int tx, int ty)
 {
     constexpr bool VISCO = WEQ == SOFI_VEL_ISO || WEQ == SOFI_VEL_VTI;
-    const int ty = t / g.ntx, tx = t - ty * g.ntx;
+    Park *const park = parks();
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
     const int i = 1 + tx * BX + threadIdx.x;
     const int j = 1 + ty * TBY + threadIdx.y;
     if (i > g.nx || j > g.ny) return;
@@ -1039,6 +1181,7 @@ __device__ __forceinline__ void stress_tile(const Grid &g, const Fields &f0, con
     const int k0 = ONE ? 0 : g.k_lo + blockIdx.y * g.spt, k1 = ONE ? 1 : min(k0 + g.spt, g.k_hi);
     for (int k = k0; k < k1; ++k) {
         Fields f = ONE ? f0 : f0.at(k, g);
+        const Frame fr = frame_load<false>(g, f, m, i, j, c, park[w]);
         float a = 0.f, b = 0.f, d = 0.f, e = 0.f;
 #pragma unroll
         for (int mm = 1; mm <= ND; ++mm) {
@@ -1049,7 +1192,7 @@ __device__ __forceinline__ void stress_tile(const Grid &g, const Fields &f0, con
             e += h * (f.vy[c + (mm - 1) * P] - f.vy[c - mm * P]);
         }
         float vxx, vyx, vxy, vyy;
-        if (!stress_dv(g, f, m, i, j, a, b, d, e, vxx, vyx, vxy, vyy)) continue;
+        if (!stress_dv(g, f, m, fr, i, j, a, b, d, e, vxx, vyx, vxy, vyy)) continue;
         float sxx = ld1<ONE>(f.sxx, c), syy = ld1<ONE>(f.syy, c),
               sxy = ld1<ONE>(f.sxy, c);
         if (WEQ == SOFI_EL_ISO) upd_el(c1, c2, c3, vxx, vyx, vxy, vyy, sxx, syy, sxy, fz, f, g.dt, c);
@@ -1085,7 +1228,7 @@ __device__ __forceinline__ void stress_tile(const Grid &g, const Fields &f0, con
             }
             visc_vti_final(g.dthalbe, c1, c2, c3, c4, sxyv, vxx, vyy, u, sxx, syy, sxy, fz, f, g.dt, c);
         }
-        stress_post<ND, VISCO>(g, f, m, s, fz, nt, i, j, c, sxx, syy, sxy);
+        stress_post<ND, VISCO>(g, f, m, s, fz, fr, nt, i, j, c, sxx, syy, sxy);
         st1<ONE>(f.sxx, c, sxx);
         st1<ONE>(f.syy, c, syy);
         st1<ONE>(f.sxy, c, sxy);
@@ -1095,7 +1238,8 @@ template <int ND, int WEQ, bool ONE>
 __global__ __launch_bounds__(BX *BY) void k_stress(Grid g, Fields f0, Mat m, Src s, Fuse fz, int nt)
 {
     if (ONE && fused_seis(g, f0, fz)) return;
-    stress_tile<ND, WEQ, ONE>(g, f0, m, s, fz, nt, tile_id());
+    const int2 t = tile_of(g, 0, 0, blockIdx.x);
+    stress_tile<ND, WEQ, ONE>(g, f0, m, s, fz, nt, t.x, t.y);
 }
 
 // VW cells per thread (see k_velocity_v); inactive cells (past NX, or
@@ -1103,7 +1247,7 @@ __global__ __launch_bounds__(BX *BY) void k_stress(Grid g, Fields f0, Mat m, Src
 // variables
 template <int ND, int WEQ, int VW, bool PRE>
 __device__ __forceinline__ void stress_v_slot(const Grid &g, Fields f, const Mat &m, const Src &s, const Fuse &fz,
-                                              int nt, int i0, int j, const vecf<VW> *pre)
+                                              int nt, int i0, int j, const vecf<VW> *pre, Park *park)
 {
     constexpr bool VISCO = WEQ == SOFI_VEL_ISO || WEQ == SOFI_VEL_VTI;
     constexpr int G = (ND + VW - 1) / VW;
@@ -1119,28 +1263,28 @@ __device__ __forceinline__ void stress_v_slot(const Grid &g, Fields f, const Mat
             yv[(q + G) * VW + k] = b[k];
         }
     }
+    // vx rows j + m and j - m + 1, vy rows j + m - 1 and j - m
+    V a1[ND], a0[ND], b1[ND], b0[ND];
+#pragma unroll
+    for (int mm = 1; mm <= ND; ++mm) {
+        a1[mm - 1] = ldv<VW>(f.vx, c0 + mm * P);
+        if (mm > 1) {
+            a0[mm - 1] = ldv<VW>(f.vx, c0 - (mm - 1) * P);
+            b1[mm - 1] = ldv<VW>(f.vy, c0 + (mm - 1) * P);
+        }
+        b0[mm - 1] = ldv<VW>(f.vy, c0 - mm * P);
+    }
+    Frame fr[VW];      // (a cell past NX fetches the neighbouring entries, which nothing uses)
+#pragma unroll
+    for (int k = 0; k < VW; ++k) fr[k] = frame_load<false>(g, f, m, i0 + k, j, c0 + k, park[k]);
     float d[VW] = {}, e[VW] = {};
 #pragma unroll
     for (int mm = 1; mm <= ND; ++mm) {
         const float h = g.hc[mm];
-        // vx rows j + m and j - m + 1, vy rows j + m - 1 and j - m
-        const V a1 = ldv<VW>(f.vx, c0 + mm * P);
-        V a0, b1;
-        if (mm == 1) {
-#pragma unroll
-            for (int k = 0; k < VW; ++k) {
-                a0[k] = xv[G * VW + k];
-                b1[k] = yv[G * VW + k];
-            }
-        } else {
-            a0 = ldv<VW>(f.vx, c0 - (mm - 1) * P);
-            b1 = ldv<VW>(f.vy, c0 + (mm - 1) * P);
-        }
-        const V b0 = ldv<VW>(f.vy, c0 - mm * P);
 #pragma unroll
         for (int k = 0; k < VW; ++k) {
-            d[k] += h * (a1[k] - a0[k]);
-            e[k] += h * (b1[k] - b0[k]);
+            d[k] += h * (a1[mm - 1][k] - (mm == 1 ? xv[G * VW + k] : a0[mm - 1][k]));
+            e[k] += h * ((mm == 1 ? yv[G * VW + k] : b1[mm - 1][k]) - b0[mm - 1][k]);
         }
     }
     float vxx[VW], vyx[VW], vxy[VW], vyy[VW];
@@ -1157,7 +1301,7 @@ __device__ __forceinline__ void stress_v_slot(const Grid &g, Fields f, const Mat
             a += h * (xv[G * VW + k + mm - 1] - xv[G * VW + k - mm]);
             b += h * (yv[G * VW + k + mm] - yv[G * VW + k - mm + 1]);
         }
-        act[k] = stress_dv(g, f, m, i0 + k, j, a, b, d[k], e[k], vxx[k], vyx[k], vxy[k], vyy[k]);
+        act[k] = stress_dv(g, f, m, fr[k], i0 + k, j, a, b, d[k], e[k], vxx[k], vyx[k], vxy[k], vyy[k]);
     }
     const V sxx0 = ldv<VW>(f.sxx, c0), syy0 = ldv<VW>(f.syy, c0), sxy0 = ldv<VW>(f.sxy, c0);
     float sxx[VW], syy[VW], sxy[VW];
@@ -1254,7 +1398,7 @@ __device__ __forceinline__ void stress_v_slot(const Grid &g, Fields f, const Mat
 #pragma unroll
     for (int k = 0; k < VW; ++k) {
         if (!act[k]) continue;
-        stress_post<ND, VISCO>(g, f, m, s, fz, nt, i0 + k, j, c0 + k, sxx[k], syy[k], sxy[k]);
+        stress_post<ND, VISCO>(g, f, m, s, fz, fr[k], nt, i0 + k, j, c0 + k, sxx[k], syy[k], sxy[k]);
         sxxn[k] = sxx[k];
         syyn[k] = syy[k];
         sxyn[k] = sxy[k];
@@ -1268,14 +1412,16 @@ __device__ __forceinline__ void stress_v_slot(const Grid &g, Fields f, const Mat
 template <int ND, int WEQ, int VW, bool ONE>
 __global__ __launch_bounds__(BX *BY) void k_stress_v(Grid g, Fields f0, Mat m, Src s, Fuse fz, int nt)
 {
+    Park(*const park)[VW] = reinterpret_cast<Park(*)[VW]>(parks());
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
     if (ONE && fused_seis(g, f0, fz)) return;
-    const int ntxv = (g.nx + BX * VW - 1) / (BX * VW);
-    const int t = tile_id(), ty = t / ntxv, tx = t - ty * ntxv;
+    const int2 t = tile_of(g, 0, VW / 2, blockIdx.x);
+    const int tx = t.x, ty = t.y;
     const int i0 = 1 + (tx * BX + threadIdx.x) * VW;
     const int j = 1 + ty * BY + threadIdx.y;
     if (i0 > g.nx || j > g.ny) return;
     if (ONE) {
-        stress_v_slot<ND, WEQ, VW, false>(g, f0, m, s, fz, nt, i0, j, nullptr);
+        stress_v_slot<ND, WEQ, VW, false>(g, f0, m, s, fz, nt, i0, j, nullptr, park[w]);
         return;
     }
     // a batch: the elastic coefficients once for the thread's slots
@@ -1294,7 +1440,7 @@ __global__ __launch_bounds__(BX *BY) void k_stress_v(Grid g, Fields f0, Mat m, S
     }
     constexpr bool P = WEQ == SOFI_EL_ISO || WEQ == SOFI_EL_VTI;
     const int k0 = g.k_lo + blockIdx.y * g.spt, k1 = min(k0 + g.spt, g.k_hi);
-    for (int k = k0; k < k1; ++k) stress_v_slot<ND, WEQ, VW, P>(g, f0.at(k, g), m, s, fz, nt, i0, j, pre);
+    for (int k = k0; k < k1; ++k) stress_v_slot<ND, WEQ, VW, P>(g, f0.at(k, g), m, s, fz, nt, i0, j, pre, park[w]);
 }
 
 // ------------------------------------ 4th order in time (Adams-Bashforth)
@@ -1323,11 +1469,15 @@ struct Hist4 {
 template <int ND>
 __global__ __launch_bounds__(BX *BY) void k_velocity4(Grid g, Fields f, Mat m, Src s, Fuse fz, int nt, Hist4 H)
 {
-    const int t = tile_id(), ty = t / g.ntx, tx = t - ty * g.ntx;
+    Park *const park = parks();
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int2 t = tile_of(g, 0, 0, blockIdx.x);
+    const int tx = t.x, ty = t.y;
     const int i = 1 + tx * BX + threadIdx.x;
     const int j = 1 + ty * BY + threadIdx.y;
     if (i > g.nx || j > g.ny) return;
     const int c = IDX(g, i, j);
+    const Frame fr = frame_load<true>(g, f, m, i, j, c, park[w]);
     const float rip = m.rip[c], rjp = m.rjp[c];
     float sxx_x, sxy_x, sxy_y, syy_y;
     op_v<ND>(g, f.sxx, f.syy, f.sxy, c, sxx_x, sxy_x, sxy_y, syy_y);
@@ -1335,11 +1485,11 @@ __global__ __launch_bounds__(BX *BY) void k_velocity4(Grid g, Fields f, Mat m, S
     if (i == g.nx / 2 && j == g.ny / 2 && isnan(vy) && *f.unstable == 0) *f.unstable = step_of(fz.ntb, nt);
     for (int k = 0; k < fz.nforce; ++k)
         if (c == fz.c[k]) force_add(g, s, fz.soff + k, step_of(fz.ntb, nt), rip, rjp, vx, vy);
-    const bool xf = in_xframe(g, i), yf = in_yframe(g, j), frame = xf || yf;
+    const bool frame = fr.any();
     bool upd = !frame || g.abs_type == 2;
     if (frame && g.abs_type == 1) {
-        cpml_v(g, f, m, i, j, xf, yf, sxx_x, sxy_x, sxy_y, syy_y);
-        upd = i > g.gx2 && !(i > g.gx3 && yf);     // right side, top and bottom only
+        cpml_v(g, f, m, fr, i, j, sxx_x, sxy_x, sxy_y, syy_y);
+        upd = i > g.gx2 && !(i > g.gx3 && fr.yf);     // right side, top and bottom only
     }
     if (upd) {
         const float sx = sxx_x + sxy_y, sy = sxy_x + syy_y;
@@ -1347,12 +1497,10 @@ __global__ __launch_bounds__(BX *BY) void k_velocity4(Grid g, Fields f, Mat m, S
         H.sy[0][c] = sy;
         vx += (AB1 * sx + AB2 * H.sx[1][c] + AB3 * H.sx[2][c] + AB4 * H.sx[3][c]) * g.dtdh * rip;
         vy += (AB1 * sy + AB2 * H.sy[1][c] + AB3 * H.sy[2][c] + AB4 * H.sy[3][c]) * g.dtdh * rjp;
-        if (frame) {     // ABS_TYPE 2: damping (abs_update_v, src/abs_update.c:46-50)
-            if (g.abs_type == 2) {
-                const float a = m.absorb[c];
-                vx *= a;
-                vy *= a;
-            }
+        if (frame && g.abs_type == 2) {     // damping (abs_update_v, src/abs_update.c:46-50)
+            const float a = m.absorb[c];
+            vx *= a;
+            vy *= a;
         }
     }
     f.vx[c] = vx;
@@ -1370,12 +1518,16 @@ __global__ __launch_bounds__(BX *BY) void k_velocity4(Grid g, Fields f, Mat m, S
 template <int ND, bool VISCO>
 __global__ __launch_bounds__(BX *BY) void k_stress4(Grid g, Fields f, Mat m, Src s, Fuse fz, int nt, Hist4 H)
 {
+    Park *const park = parks();
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
     if (fused_seis(g, f, fz)) return;
-    const int t = tile_id(), ty = t / g.ntx, tx = t - ty * g.ntx;
+    const int2 t = tile_of(g, 0, 0, blockIdx.x);
+    const int tx = t.x, ty = t.y;
     const int i = 1 + tx * BX + threadIdx.x;
     const int j = 1 + ty * BY + threadIdx.y;
     if (i > g.nx || j > g.ny) return;
     const int c = IDX(g, i, j), P = g.pitch;
+    const Frame fr = frame_load<false>(g, f, m, i, j, c, park[w]);
     float a = 0.f, b = 0.f, d = 0.f, e = 0.f;
 #pragma unroll
     for (int mm = 1; mm <= ND; ++mm) {
@@ -1386,7 +1538,7 @@ __global__ __launch_bounds__(BX *BY) void k_stress4(Grid g, Fields f, Mat m, Src
         e += h * (f.vy[c + (mm - 1) * P] - f.vy[c - mm * P]);
     }
     float vxx, vyx, vxy, vyy;
-    if (!stress_dv(g, f, m, i, j, a, b, d, e, vxx, vyx, vxy, vyy)) return;
+    if (!stress_dv(g, f, m, fr, i, j, a, b, d, e, vxx, vyx, vxy, vyy)) return;
     const float dhi = g.dhi4;
     const float cur[4] = { vxx * g.dh, vyy * g.dh, vxy * g.dh, vyx * g.dh };
     float sum[4];
@@ -1443,7 +1595,7 @@ __global__ __launch_bounds__(BX *BY) void k_stress4(Grid g, Fields f, Mat m, Src
     sxy += u1;
     sxx += u2;
     syy += u3;
-    stress_post<ND, VISCO>(g, fo, m, s, fz, nt, i, j, c, sxx, syy, sxy);
+    stress_post<ND, VISCO>(g, fo, m, s, fz, fr, nt, i, j, c, sxx, syy, sxy);
     f.sxx[c] = sxx;
     f.syy[c] = syy;
     f.sxy[c] = sxy;
@@ -1462,9 +1614,8 @@ __global__ __launch_bounds__(BX *BY) void k_stress4(Grid g, Fields f, Mat m, Src
 // and to syy).
 template <int ND, bool ONE, int TBY = BY>
 __device__ __forceinline__ void stress_ac_tile(const Grid &g, const Fields &f0, const Mat &m, const Src &s,
-                                               const Fuse &fz, int nt, int t)
+                                               const Fuse &fz, int nt, int tx, int ty)
 {
-    const int ty = t / g.ntx, tx = t - ty * g.ntx;
     const int i = 1 + tx * BX + threadIdx.x;
     const int j = 1 + ty * TBY + threadIdx.y;
     if (i > g.nx || j > g.ny) return;
@@ -1514,7 +1665,8 @@ template <int ND, bool ONE>
 __global__ __launch_bounds__(BX *BY) void k_stress_ac(Grid g, Fields f0, Mat m, Src s, Fuse fz, int nt)
 {
     if (ONE && fused_seis(g, f0, fz)) return;
-    stress_ac_tile<ND, ONE>(g, f0, m, s, fz, nt, tile_id());
+    const int2 t = tile_of(g, 0, 0, blockIdx.x);
+    stress_ac_tile<ND, ONE>(g, f0, m, s, fz, nt, t.x, t.y);
 }
 
 // ------------------------------------------------------ work-list launches
@@ -1550,9 +1702,9 @@ __global__ __launch_bounds__(BX *TBY) void k_velocity_w(const Shot *__restrict__
     for (int w = blockIdx.x; w < n; w += gridDim.x) {
         const int2 e = item[w];
         const Shot &d = sh[e.x];
-        const int last = d.g.ntx * ((d.g.ny + TBY - 1) / TBY);
-        for (int r = 0, t = e.y; r < rows && t < last; ++r, t += d.g.ntx)
-            velocity_tile<ND, true, NT, TBY>(d.g, d.f, d.m, d.s, d.fv, it, t);
+        const int ty0 = div_by(d.g.tdiv[0], e.y), tx = e.y - ty0 * d.g.ntx;
+        const int last = min(ty0 + rows, (d.g.ny + TBY - 1) / TBY);
+        for (int ty = ty0; ty < last; ++ty) velocity_tile<ND, true, NT, TBY>(d.g, d.f, d.m, d.s, d.fv, it, tx, ty);
     }
 }
 
@@ -1593,10 +1745,11 @@ __global__ __launch_bounds__(BX *TBY) void k_stress_w(const Shot *__restrict__ s
     for (int w = blockIdx.x; w < n; w += gridDim.x) {
         const int2 e = item[w];
         const Shot &d = sh[e.x];
-        const int last = d.g.ntx * ((d.g.ny + TBY - 1) / TBY);
-        for (int r = 0, t = e.y; r < rows && t < last; ++r, t += d.g.ntx) {
-            if constexpr (WEQ == SOFI_AC_ISO) stress_ac_tile<ND, true, TBY>(d.g, d.f, d.m, d.s, d.fs, it, t);
-            else stress_tile<ND, WEQ, true, TBY>(d.g, d.f, d.m, d.s, d.fs, it, t);
+        const int ty0 = div_by(d.g.tdiv[0], e.y), tx = e.y - ty0 * d.g.ntx;
+        const int last = min(ty0 + rows, (d.g.ny + TBY - 1) / TBY);
+        for (int ty = ty0; ty < last; ++ty) {
+            if constexpr (WEQ == SOFI_AC_ISO) stress_ac_tile<ND, true, TBY>(d.g, d.f, d.m, d.s, d.fs, it, tx, ty);
+            else stress_tile<ND, WEQ, true, TBY>(d.g, d.f, d.m, d.s, d.fs, it, tx, ty);
         }
     }
 }
@@ -1822,7 +1975,10 @@ __global__ void k_wrap_x(Grid g, float *a, float *b)
 template <int ND, int S>
 __global__ __launch_bounds__(BX *BY) void k_velocity_b(Grid g, Fields f0, Mat m, int nt, const int *ntb, int fwi_acc)
 {
-    const int t = blockIdx.x, ty = t / g.ntx, tx = t - ty * g.ntx;
+    Park(*const park)[S] = reinterpret_cast<Park(*)[S]>(parks());
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int2 t = tile_of(g, 0, 0, blockIdx.x);
+    const int tx = t.x, ty = t.y;
     const int i = 1 + tx * BX + threadIdx.x;
     const int j = 1 + ty * BY + threadIdx.y;
     if (i > g.nx || j > g.ny) return;
@@ -1830,9 +1986,11 @@ __global__ __launch_bounds__(BX *BY) void k_velocity_b(Grid g, Fields f0, Mat m,
     const float rip = m.rip[c], rjp = m.rjp[c];
     const int k0 = g.k_lo + blockIdx.y * S;
     float a[S], b[S], d[S], e[S], vx[S], vy[S];
+    Frame fr[S];
 #pragma unroll
     for (int q = 0; q < S; ++q) {
         const Fields f = f0.at(k0 + q, g);
+        fr[q] = frame_load<true>(g, f, m, i, j, c, park[w][q]);
         op_v<ND>(g, f.sxx, f.syy, f.sxy, c, a[q], b[q], d[q], e[q]);
         vx[q] = f.vx[c];
         vy[q] = f.vy[c];
@@ -1844,7 +2002,7 @@ __global__ __launch_bounds__(BX *BY) void k_velocity_b(Grid g, Fields f0, Mat m,
 #pragma unroll
     for (int q = 0; q < S; ++q) {
         Fields f = f0.at(k0 + q, g);
-        velocity_core(g, f, m, s0, fz, nt, i, j, c, a[q], b[q], d[q], e[q], rip, rjp, vx[q], vy[q]);
+        velocity_core(g, f, m, s0, fz, fr[q], nt, i, j, c, a[q], b[q], d[q], e[q], rip, rjp, vx[q], vy[q]);
         f.vx[c] = vx[q];
         f.vy[c] = vy[q];
     }
@@ -1855,7 +2013,10 @@ __global__ __launch_bounds__(BX *BY) void k_stress_b(Grid g, Fields f0, Mat m, i
                                                      PFuse pf)
 {
     constexpr bool VISCO = WEQ == SOFI_VEL_ISO || WEQ == SOFI_VEL_VTI;
-    const int t = blockIdx.x, ty = t / g.ntx, tx = t - ty * g.ntx;
+    Park(*const park)[S] = reinterpret_cast<Park(*)[S]>(parks());
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int2 t = tile_of(g, 0, 0, blockIdx.x);
+    const int tx = t.x, ty = t.y;
     const int i = 1 + tx * BX + threadIdx.x;
     const int j = 1 + ty * BY + threadIdx.y;
     if (i > g.nx || j > g.ny) return;
@@ -1885,9 +2046,11 @@ __global__ __launch_bounds__(BX *BY) void k_stress_b(Grid g, Fields f0, Mat m, i
     }
     const int k0 = g.k_lo + blockIdx.y * S;
     float a[S], b[S], d[S], e[S], sxx[S], syy[S], sxy[S];
+    Frame fr[S];
 #pragma unroll
     for (int q = 0; q < S; ++q) {
         const Fields f = f0.at(k0 + q, g);
+        fr[q] = frame_load<false>(g, f, m, i, j, c, park[w][q]);
         float a_ = 0.f, b_ = 0.f, d_ = 0.f, e_ = 0.f;
 #pragma unroll
         for (int mm = 1; mm <= ND; ++mm) {
@@ -1913,7 +2076,7 @@ __global__ __launch_bounds__(BX *BY) void k_stress_b(Grid g, Fields f0, Mat m, i
     for (int q = 0; q < S; ++q) {
         Fields f = f0.at(k0 + q, g);
         float vxx, vyx, vxy, vyy;
-        if (!stress_dv(g, f, m, i, j, a[q], b[q], d[q], e[q], vxx, vyx, vxy, vyy)) continue;
+        if (!stress_dv(g, f, m, fr[q], i, j, a[q], b[q], d[q], e[q], vxx, vyx, vxy, vyy)) continue;
         float sx = sxx[q], sy = syy[q], sz = sxy[q];
         if (WEQ == SOFI_EL_ISO) upd_el(c1, c2, c3, vxx, vyx, vxy, vyy, sx, sy, sz, fz, f, g.dt, c);
         if (WEQ == SOFI_EL_VTI) upd_el_vti(c1, c2, c3, c4, vxx, vyx, vxy, vyy, sx, sy, sz, fz, f, g.dt, c);
@@ -1947,7 +2110,7 @@ __global__ __launch_bounds__(BX *BY) void k_stress_b(Grid g, Fields f0, Mat m, i
             }
             visc_vti_final(g.dthalbe, c1, c2, c3, c4, sxyv, vxx, vyy, u, sx, sy, sz, fz, f, g.dt, c);
         }
-        stress_post<ND, VISCO>(g, f, m, s0, fz, nt, i, j, c, sx, sy, sz);
+        stress_post<ND, VISCO>(g, f, m, s0, fz, fr[q], nt, i, j, c, sx, sy, sz);
         for (int w = 0; w < pf.n; ++w)
             if (pf.k[w] == k0 + q && pf.c[w] == c) {
                 const float amp = psource_amp(g, s, pf.l[w], step_of(ntb, nt));
@@ -1984,13 +2147,22 @@ template <int ND, int WEQ, int S>
 __global__ __launch_bounds__(BX *BY) void k_stress_tti_f(Grid g, Fields f0, Mat m, Fuse fz, Src src, int nt)
 {
     constexpr int LX = BX + 2, LY = BY + 2;
+    Park(*const park)[S] = reinterpret_cast<Park(*)[S]>(parks());
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
     __shared__ float sd[S][4][LY][LX];   // dvxx, dvyy, dvyx, dvxy of rows j0-1..j0+BY, columns i0-1..i0+BX
-    const int t = blockIdx.x, ty = t / g.ntx, tx = t - ty * g.ntx;
+    // (tiles in plain order: the frame's rows first made one EL_TTI shot 1 % slower)
+    const int ty = div_by(g.tdiv[0], blockIdx.x), tx = blockIdx.x - ty * g.ntx;
     const int i0 = 1 + tx * BX, j0 = 1 + ty * BY;
     const int k0 = g.k_lo + blockIdx.y * S;
     const bool cpml = g.abs_type == 1 && g.fw > 0;
     const bool store_dv = cpml && is_frame_tile(g, tx, ty);
     const int tid = threadIdx.y * BX + threadIdx.x;
+    const int i = i0 + threadIdx.x, j = j0 + threadIdx.y;
+    Frame fr[S];
+    if (store_dv && i <= g.nx && j <= g.ny) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) fr[s] = frame_load<false>(g, f0.at(k0 + s, g), m, i, j, IDX(g, i, j), park[w][s]);
+    }
     for (int q = tid; q < LX * LY; q += BX * BY) {
         const int lj = q / LX, li = q - lj * LX;
         const int ii = i0 - 1 + li, jj = j0 - 1 + lj;
@@ -2028,7 +2200,6 @@ __global__ __launch_bounds__(BX *BY) void k_stress_tti_f(Grid g, Fields f0, Mat 
         }
     }
     __syncthreads();
-    const int i = i0 + threadIdx.x, j = j0 + threadIdx.y;
     if (i > g.nx || j > g.ny) return;
     const int c = IDX(g, i, j);
     const int li = threadIdx.x + 1, lj = threadIdx.y + 1;
@@ -2043,7 +2214,7 @@ __global__ __launch_bounds__(BX *BY) void k_stress_tti_f(Grid g, Fields f0, Mat 
             for (int s = 0; s < S; ++s) {
                 Fields f = f0.at(k0 + s, g);
                 float vxx = sd[s][0][lj][li], vyy = sd[s][1][lj][li], vyx = sd[s][2][lj][li], vxy = sd[s][3][lj][li];
-                if (!tti_cpml_skipped(g, i, j)) cpml_dv(g, m, f, i, j, xf, yf, vxx, vyx, vxy, vyy);
+                if (!tti_cpml_skipped(g, i, j)) cpml_dv(g, m, f, fr[s], i, j, vxx, vyx, vxy, vyy);
                 f.dvxx[c] = vxx;
                 f.dvyy[c] = vyy;
                 f.dvyx[c] = vyx;
@@ -2436,7 +2607,8 @@ struct sofi_dev {
     // device-side copies owned by the handle
     float *mat[SOFI_A_NARRAYS] = {};
     float *base_d = nullptr, *base_e = nullptr, *base_r = nullptr;
-    float *prof = nullptr;
+    float *prof = nullptr, *pml = nullptr;
+    int kone = 0;
     float *surf = nullptr;
     // acquisition of every shot slot (host copies); combined into the device
     // lists Src / Rec by sync_acq before the next time step
@@ -2765,6 +2937,12 @@ int sofi_open_batch(const sofi_desc *desc, int nshots, sofi_dev **out)
     g.wy = d.nx + 1;
     g.ntx = (d.nx + BX - 1) / BX;
     g.nty = (d.ny + BY - 1) / BY;
+    for (int k = 0; k < 2; ++k) {
+        const int rows = k ? VROWS * BY : BY;
+        g.low[k].first = std::min(d.gy[3], d.ny - 1) / rows;
+        g.low[k].n = (d.ny + rows - 1) / rows - g.low[k].first;
+    }
+    for (int k = 0; k < 3; ++k) g.tdiv[k] = fast_div((d.nx + (BX << k) - 1) / (BX << k));
     g.periodic = d.boundary == 1;
     frame_tiles(g);
     g.nxp = (d.ny + 1) * g.wx;
@@ -2944,6 +3122,16 @@ int sofi_set_medium(sofi_dev *h, const float *const *arrays, const float *const 
             memcpy(pr.data() + (size_t)k * n, profiles[k], n * sizeof(float));
         }
         if (upload(h, &h->prof, pr.data(), pr.size())) return -1;
+        std::vector<float> tab((size_t)8 * n);
+        h->kone = 1;
+        for (int side = 0; side < 2; ++side)
+            for (int k = 0; k < n; ++k) {
+                const float *q = pr.data() + (size_t)(side ? SOFI_P_K_Y : SOFI_P_K_X) * n + k;   // K, a, b, then at half points
+                const float row[4] = { q[2 * n], q[n], q[5 * n], q[4 * n] };
+                memcpy(tab.data() + 4 * ((size_t)side * n + k), row, sizeof(row));
+                if (k > 0 && (q[0] != 1.0f || q[3 * n] != 1.0f)) h->kone = 0;
+            }
+        if (upload(h, &h->pml, tab.data(), tab.size())) return -1;
     }
     m = Mat();
     m.rip = h->mat[SOFI_A_RIP];
@@ -2984,6 +3172,9 @@ int sofi_set_medium(sofi_dev *h, const float *const *arrays, const float *const 
     m.ptaus = h->mat[SOFI_A_PTAUS];
     m.ptaup = h->mat[SOFI_A_PTAUP];
     m.prof = h->prof;
+    m.pmlx = reinterpret_cast<decltype(m.pmlx)>(h->pml);
+    m.pmly = m.pmlx ? m.pmlx + (2 * d.fw + 1) : nullptr;
+    m.kone = h->kone;
     if (d.free_surf) {
         // row-1 coefficients of the free surface (see SURF_*)
         const float *pu = arrays[SOFI_A_PU], *ppi = arrays[SOFI_A_PPI];
@@ -3393,19 +3584,19 @@ void rot4(float **v)
 // one (graphs are built node by node, not by stream capture, so other
 // threads' synchronous HIP calls cannot invalidate a recording)
 template <typename... P, typename... A>
-void launch(sofi_dev *h, void (*k)(P...), dim3 grid, dim3 block, A &&...a)
+void launch_lds(sofi_dev *h, void (*k)(P...), dim3 grid, dim3 block, size_t lds, A &&...a)
 {
     using Tup = std::tuple<std::decay_t<P>...>;
     if (h->defer) {
         // a step recorded for the work-list launches: issued later, in its stage
         auto v = std::make_shared<Tup>(std::forward<A>(a)...);
-        h->defer->push_back({h->dstage, [k, grid, block, v](hipStream_t st) {
+        h->defer->push_back({h->dstage, [k, grid, block, lds, v](hipStream_t st) {
             void *args[sizeof...(P) > 0 ? sizeof...(P) : 1];
             std::apply([&](auto &...x) {
                 int q = 0;
                 ((args[q++] = (void *)&x), ...);
             }, *v);
-            return hipLaunchKernel(reinterpret_cast<const void *>(k), grid, block, args, 0, st);
+            return hipLaunchKernel(reinterpret_cast<const void *>(k), grid, block, args, lds, st);
         }});
         return;
     }
@@ -3417,7 +3608,7 @@ void launch(sofi_dev *h, void (*k)(P...), dim3 grid, dim3 block, A &&...a)
             ((args[q++] = (void *)&x), ...);
         }, v);
         const hipError_t e =
-            hipLaunchKernel(reinterpret_cast<const void *>(k), grid, block, args, 0, h->cur ? h->cur : h->stream);
+            hipLaunchKernel(reinterpret_cast<const void *>(k), grid, block, args, lds, h->cur ? h->cur : h->stream);
         if (e != hipSuccess && h->gerr == hipSuccess) h->gerr = e;
         return;
     }
@@ -3436,7 +3627,7 @@ void launch(sofi_dev *h, void (*k)(P...), dim3 grid, dim3 block, A &&...a)
     p.func = reinterpret_cast<void *>(k);
     p.gridDim = grid;
     p.blockDim = block;
-    p.sharedMemBytes = 0;
+    p.sharedMemBytes = (unsigned)lds;
     p.kernelParams = h->gargs.back().ptrs.data();
     p.extra = nullptr;
     hipGraphNode_t n = nullptr;
@@ -3446,6 +3637,19 @@ void launch(sofi_dev *h, void (*k)(P...), dim3 grid, dim3 block, A &&...a)
     } else {
         h->glast = n;
     }
+}
+
+template <typename... P, typename... A>
+void launch(sofi_dev *h, void (*k)(P...), dim3 grid, dim3 block, A &&...a)
+{
+    launch_lds(h, k, grid, block, 0, std::forward<A>(a)...);
+}
+
+// LDS of an update kernel's frame fetches: a Park for each of a block's
+// `waves` waves and `cells` cells per thread
+size_t park_bytes(const Grid &g, int cells, int waves = BY)
+{
+    return g.abs_type == 1 && g.fw > 0 ? sizeof(Park) * (size_t)waves * (size_t)cells : 0;
 }
 
 // the periodic wrap of the ghost columns of a (vx / sxy position) and b (vy
@@ -3484,15 +3688,15 @@ void launch_blocks(sofi_dev *h, Grid gg, int lo, int hi, int S, A &&...a)
     if (n > 0) {
         gg.k_lo = lo;
         gg.k_hi = lo + n * S;
-        if (S == 4) launch(h, K<4>::fn(), dim3(ntile, n), blk, gg, a...);
-        else if (S == 2) launch(h, K<2>::fn(), dim3(ntile, n), blk, gg, a...);
-        else launch(h, K<1>::fn(), dim3(ntile, n), blk, gg, a...);
+        if (S == 4) launch_lds(h, K<4>::fn(), dim3(ntile, n), blk, park_bytes(gg, 4), gg, a...);
+        else if (S == 2) launch_lds(h, K<2>::fn(), dim3(ntile, n), blk, park_bytes(gg, 2), gg, a...);
+        else launch_lds(h, K<1>::fn(), dim3(ntile, n), blk, park_bytes(gg, 1), gg, a...);
     }
     const int r0 = lo + n * S;
     if (r0 < hi && S != 1) {
         gg.k_lo = r0;
         gg.k_hi = hi;
-        launch(h, K<1>::fn(), dim3(ntile, hi - r0), blk, gg, a...);
+        launch_lds(h, K<1>::fn(), dim3(ntile, hi - r0), blk, park_bytes(gg, 1), gg, a...);
     }
 }
 template <int ND>
@@ -3637,7 +3841,7 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
             // update (src/time_loop.c:89-91,226-244); the memory variables
             // the rest of the step sees are the ones just written
             const dim3 t4((g.nx + BX - 1) / BX * nty);
-            launch(h, k_velocity4<ND>, t4, blk, gg, f, m, h->s, fv, nt, h->h4);
+            launch_lds(h, k_velocity4<ND>, t4, blk, park_bytes(g, 1), gg, f, m, h->s, fv, nt, h->h4);
             wrap_x(h, gg, lo, gg.k_hi, f.vx, f.vy);
             rot4(h->h4.sx);
             rot4(h->h4.sy);
@@ -3655,8 +3859,8 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
                 fss.rec = rr;
                 ts.x += fss.sblk;
             }
-            if (g.L > 0) launch(h, k_stress4<ND, true>, ts, blk, gg, f, m, h->s, fss, nt, h->h4);
-            else launch(h, k_stress4<ND, false>, ts, blk, gg, f, m, h->s, fss, nt, h->h4);
+            if (g.L > 0) launch_lds(h, k_stress4<ND, true>, ts, blk, park_bytes(g, 1), gg, f, m, h->s, fss, nt, h->h4);
+            else launch_lds(h, k_stress4<ND, false>, ts, blk, park_bytes(g, 1), gg, f, m, h->s, fss, nt, h->h4);
             for (int q = 0; q < 4; ++q) rot4(h->h4.dv[q]);
             if (g.L > 0) {
                 rot4(h->h4.r);
@@ -3726,13 +3930,13 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
             h->wl_shot.r = h->r;
             h->wl_shot.seismo = d.seismo;
             h->dstage = 1;
-        } else if (vw == 4 && one) launch(h, k_velocity_v<ND, 4, true>, tiles, blk, gg, fk, m, h->s, fv_l, nt);
-        else if (vw == 4) launch(h, k_velocity_v<ND, 4, false>, tiles, blk, gg, fk, m, h->s, fv_l, nt);
-        else if (vw == 2 && one) launch(h, k_velocity_v<ND, 2, true>, tiles, blk, gg, fk, m, h->s, fv_l, nt);
-        else if (vw == 2) launch(h, k_velocity_v<ND, 2, false>, tiles, blk, gg, fk, m, h->s, fv_l, nt);
-        else if (one && tti) launch(h, k_velocity<ND, true, false>, tiles, blk, gg, fk, m, h->s, fv_l, nt);
-        else if (one) launch(h, k_velocity_r<ND, true, VROWS>, vtiles, blk, gg, fk, m, h->s, fv_l, nt);
-        else launch(h, k_velocity<ND, false>, tiles, blk, gg, fk, m, h->s, fv_l, nt);
+        } else if (vw == 4 && one) launch_lds(h, k_velocity_v<ND, 4, true>, tiles, blk, park_bytes(g, 4), gg, fk, m, h->s, fv_l, nt);
+        else if (vw == 4) launch_lds(h, k_velocity_v<ND, 4, false>, tiles, blk, park_bytes(g, 4), gg, fk, m, h->s, fv_l, nt);
+        else if (vw == 2 && one) launch_lds(h, k_velocity_v<ND, 2, true>, tiles, blk, park_bytes(g, 2), gg, fk, m, h->s, fv_l, nt);
+        else if (vw == 2) launch_lds(h, k_velocity_v<ND, 2, false>, tiles, blk, park_bytes(g, 2), gg, fk, m, h->s, fv_l, nt);
+        else if (one && tti) launch_lds(h, k_velocity<ND, true, false>, tiles, blk, park_bytes(g, 1), gg, fk, m, h->s, fv_l, nt);
+        else if (one) launch_lds(h, k_velocity_r<ND, true, VROWS>, vtiles, blk, park_bytes(g, VROWS), gg, fk, m, h->s, fv_l, nt);
+        else launch_lds(h, k_velocity<ND, false>, tiles, blk, park_bytes(g, 1), gg, fk, m, h->s, fv_l, nt);
         wrap_x(h, gg, lo, gg.k_hi, f.vx, f.vy);
         vw = vec_width(g, h->shape_s);
         tiles = dim3((g.nx + BX * vw - 1) / (BX * vw) * nty, nchunk);
@@ -3758,12 +3962,12 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
         }
 #define SOFI_STRESS(W)                                                                                      \
         do {                                                                                                \
-            if (vw == 4 && one) launch(h, k_stress_v<ND, W, 4, true>, tiles, blk, gg, fk, m, h->s, fss, nt);   \
-            else if (vw == 4) launch(h, k_stress_v<ND, W, 4, false>, tiles, blk, gg, fk, m, h->s, fss, nt);    \
-            else if (vw == 2 && one) launch(h, k_stress_v<ND, W, 2, true>, tiles, blk, gg, fk, m, h->s, fss, nt);   \
-            else if (vw == 2) launch(h, k_stress_v<ND, W, 2, false>, tiles, blk, gg, fk, m, h->s, fss, nt);    \
-            else if (one) launch(h, k_stress<ND, W, true>, tiles, blk, gg, fk, m, h->s, fss, nt);              \
-            else launch(h, k_stress<ND, W, false>, tiles, blk, gg, fk, m, h->s, fss, nt);            \
+            if (vw == 4 && one) launch_lds(h, k_stress_v<ND, W, 4, true>, tiles, blk, park_bytes(g, 4), gg, fk, m, h->s, fss, nt);   \
+            else if (vw == 4) launch_lds(h, k_stress_v<ND, W, 4, false>, tiles, blk, park_bytes(g, 4), gg, fk, m, h->s, fss, nt);    \
+            else if (vw == 2 && one) launch_lds(h, k_stress_v<ND, W, 2, true>, tiles, blk, park_bytes(g, 2), gg, fk, m, h->s, fss, nt);   \
+            else if (vw == 2) launch_lds(h, k_stress_v<ND, W, 2, false>, tiles, blk, park_bytes(g, 2), gg, fk, m, h->s, fss, nt);    \
+            else if (one) launch_lds(h, k_stress<ND, W, true>, tiles, blk, park_bytes(g, 1), gg, fk, m, h->s, fss, nt);              \
+            else launch_lds(h, k_stress<ND, W, false>, tiles, blk, park_bytes(g, 1), gg, fk, m, h->s, fss, nt);            \
         } while (0)
         if (h->wl) {
             h->wl_shot.fs = fss;
@@ -4578,20 +4782,21 @@ int many_items(ManyCtx &c, int rows, int waves)
 
 // one update launch of a work-list step in tiles of BX x TBY cells
 template <int ND, int TBY>
-void many_launch(hipStream_t st, int weq, bool stress, unsigned grid, const Shot *tab, const int2 *item, int n,
-                 int rows, int it)
+void many_launch(hipStream_t st, int weq, bool stress, unsigned grid, bool pml, const Shot *tab, const int2 *item,
+                 int n, int rows, int it)
 {
     const dim3 blk(BX, TBY);
+    const size_t lds = pml ? sizeof(Park) * TBY : 0;       // see park_bytes
     if (!stress) {
-        hipLaunchKernelGGL((k_velocity_w<ND, true, TBY>), dim3(grid), blk, 0, st, tab, item, n, rows, it);
+        hipLaunchKernelGGL((k_velocity_w<ND, true, TBY>), dim3(grid), blk, lds, st, tab, item, n, rows, it);
         return;
     }
     switch (weq) {
-      case SOFI_EL_ISO: hipLaunchKernelGGL((k_stress_w<ND, SOFI_EL_ISO, TBY>), dim3(grid), blk, 0, st, tab, item, n, rows, it); break;
-      case SOFI_VEL_ISO: hipLaunchKernelGGL((k_stress_w<ND, SOFI_VEL_ISO, TBY>), dim3(grid), blk, 0, st, tab, item, n, rows, it); break;
-      case SOFI_EL_VTI: hipLaunchKernelGGL((k_stress_w<ND, SOFI_EL_VTI, TBY>), dim3(grid), blk, 0, st, tab, item, n, rows, it); break;
-      case SOFI_AC_ISO: hipLaunchKernelGGL((k_stress_w<ND, SOFI_AC_ISO, TBY>), dim3(grid), blk, 0, st, tab, item, n, rows, it); break;
-      default: hipLaunchKernelGGL((k_stress_w<ND, SOFI_VEL_VTI, TBY>), dim3(grid), blk, 0, st, tab, item, n, rows, it);
+      case SOFI_EL_ISO: hipLaunchKernelGGL((k_stress_w<ND, SOFI_EL_ISO, TBY>), dim3(grid), blk, lds, st, tab, item, n, rows, it); break;
+      case SOFI_VEL_ISO: hipLaunchKernelGGL((k_stress_w<ND, SOFI_VEL_ISO, TBY>), dim3(grid), blk, lds, st, tab, item, n, rows, it); break;
+      case SOFI_EL_VTI: hipLaunchKernelGGL((k_stress_w<ND, SOFI_EL_VTI, TBY>), dim3(grid), blk, lds, st, tab, item, n, rows, it); break;
+      case SOFI_AC_ISO: hipLaunchKernelGGL((k_stress_w<ND, SOFI_AC_ISO, TBY>), dim3(grid), blk, lds, st, tab, item, n, rows, it); break;
+      default: hipLaunchKernelGGL((k_stress_w<ND, SOFI_VEL_VTI, TBY>), dim3(grid), blk, lds, st, tab, item, n, rows, it);
     }
 }
 
@@ -4639,10 +4844,12 @@ int many_step(ManyCtx &c, int k, ManyCfg cfg)
     };
     auto update = [&](bool stress) {
         const int weq = c.hs[0]->d.weq;
+        bool pml = false;
+        for (const sofi_dev *h : c.hs) pml = pml || park_bytes(h->g, 1) > 0;
         switch (cfg.waves) {
-          case 2: many_launch<ND, 2>(c.st, weq, stress, grid, c.dtab, c.ditem, nit, cfg.rows, k + 1); break;
-          case 8: many_launch<ND, 8>(c.st, weq, stress, grid, c.dtab, c.ditem, nit, cfg.rows, k + 1); break;
-          default: many_launch<ND, 4>(c.st, weq, stress, grid, c.dtab, c.ditem, nit, cfg.rows, k + 1);
+          case 2: many_launch<ND, 2>(c.st, weq, stress, grid, pml, c.dtab, c.ditem, nit, cfg.rows, k + 1); break;
+          case 8: many_launch<ND, 8>(c.st, weq, stress, grid, pml, c.dtab, c.ditem, nit, cfg.rows, k + 1); break;
+          default: many_launch<ND, 4>(c.st, weq, stress, grid, pml, c.dtab, c.ditem, nit, cfg.rows, k + 1);
         }
     };
     // the samplers of every handle that samples in this step, one launch each
@@ -5016,7 +5223,7 @@ size_t sofi_estimate_footprint(const sofi_desc *d, int nshots, int ntr, int nsna
     }
     if (d->abs_type == 2 && d->fw > 0) arrays += 1;
     b += arrays * (pl + A);
-    if (d->abs_type == 1 && d->fw > 0) b += 12 * wx * 4 + A;
+    if (d->abs_type == 1 && d->fw > 0) b += 20 * wx * 4 + 2 * A;
     if (d->free_surf) b += 5 * (size_t)d->nx * 4 + A;
     const size_t ns = (size_t)(d->ns > 0 ? d->ns : 1), nr = (size_t)(ntr > 0 ? ntr : 0) * nb;
     b += (SOFI_NCOMP * nr * ns * 4 + A) + (nr * 3 * 4 + A) + (nr * 2 * 8 + A) + (nr * 3 * 8 + A);
