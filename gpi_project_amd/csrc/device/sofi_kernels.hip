@@ -85,6 +85,8 @@ struct Grid {
     FastDiv tdiv[3];    // division by the tiles per row of the shapes of 1, 2 and 4 cells per thread
     // tile rows of the lower absorbing frame, in tiles of BY and of VROWS BY rows
     struct { int first, n; } low[2];
+    int nvtile;         // tiles of VROWS BY rows
+    bool fma;           // EL_ISO: see upd_el
     int wx, wy;     // row lengths of x-frame and y-frame CPML memory
     int ntx;        // tiles along x of the one-cell-per-thread update kernels
     int nty;        // tiles along y of the same
@@ -782,17 +784,16 @@ __device__ __forceinline__ void velocity_core(const Grid &g, Fields &f, const Ma
     }
 }
 
-// In the one-shot kernels (ONE), arrays that a kernel touches only at the cell
-// itself (vx, vy, rip, rjp here; the stresses, memory variables and
+// In the one-shot kernels (ONE) with NT, arrays that a kernel touches only at
+// the cell itself (vx, vy, rip, rjp here; the stresses, memory variables and
 // coefficients in k_stress) are read and written with nontemporal hints, so
 // that they stream past the L2 and leave it to the stencil arrays' rows, which
-// neighbouring tiles read again (viscoelastic FD8 on 4000 x 2000: 9 % less time
-// per step, stress kernel 72 -> 77 % of 8 TB/s).  The vector-shape kernels of
-// the elastic rheologies ran slower with the same hints (-17 % for a batch of
-// EL_VTI shots on 2000 x 1000) and keep plain accesses, and so does the
-// velocity kernel of the TTI rheologies (NT false: the TTI stress kernel
-// reads vx, vy right after for its derivatives; with the hints one EL_TTI
-// shot on 2000 x 1000 ran 11 % slower).
+// neighbouring tiles read again.  It pays where a step's data is more than the
+// caches hold (see NT_BYTES for the line and both sides' rates).  The
+// vector-shape kernels keep plain accesses (-17 % for a batch of EL_VTI shots on
+// 2000 x 1000), and so does the velocity kernel of the TTI rheologies (the TTI
+// stress kernel reads vx, vy right after for its derivatives; with the hints
+// one EL_TTI shot on 2000 x 1000 ran 11 % slower).
 //
 // one thread per cell; blockIdx.y picks g.spt shot slots of a batch, which
 // the thread updates in turn with the cell's coefficients read once (ONE: the
@@ -994,15 +995,17 @@ __device__ __forceinline__ void fwi_u_store(const Fuse &fz, const Fields &f, flo
     }
 }
 
-// wavefield_update_s_el (src/wavefield_update_s_el.c:28-48)
-__device__ __forceinline__ void upd_el(float f_, float g_, float fipjp, float vxx, float vyx, float vxy, float vyy,
-                                       float &sxx, float &syy, float &sxy, const Fuse &fz, const Fields &f, float dt, int c)
+// wavefield_update_s_el (src/wavefield_update_s_el.c:28-48).  one: the shear
+// increment is added with one rounding, as the vector shapes do and with them
+// the automatic shape (Grid::fma)
+__device__ __forceinline__ void upd_el(bool one, float f_, float g_, float fipjp, float vxx, float vyx, float vxy,
+                                       float vyy, float &sxx, float &syy, float &sxy, const Fuse &fz, const Fields &f, float dt, int c)
 {
     const float u1 = fipjp * (vyx + vxy);
     const float ff = 2.0f * f_;
     const float u2 = (g_ * (vxx + vyy)) - (ff * vyy);
     const float u3 = (g_ * (vxx + vyy)) - (ff * vxx);
-    sxy += u1;
+    sxy = one ? __builtin_fmaf(fipjp, vyx + vxy, sxy) : sxy + u1;
     sxx += u2;
     syy += u3;
     fwi_u_store(fz, f, dt, c, u1, u2, u3);
@@ -1142,7 +1145,7 @@ __device__ __forceinline__ void stress_post(const Grid &g, Fields &f, const Mat 
 // blockIdx.y picks g.spt shot slots of a batch, updated in turn with the
 // cell's material coefficients read once (ONE: a one-shot handle's single
 // slot, as in k_velocity).
-template <int ND, int WEQ, bool ONE, int TBY = BY>
+template <int ND, int WEQ, bool ONE, bool NT, int TBY = BY>
 __device__ __forceinline__ void stress_tile(const Grid &g, const Fields &f0, const Mat &m, const Src &s,
                                             const Fuse &fz, int nt, int tx, int ty)
 {
@@ -1157,14 +1160,14 @@ __device__ __forceinline__ void stress_tile(const Grid &g, const Fields &f0, con
     // EL_VTI c11 c13 c33 c55ipjp; VEL_VTI the unrelaxed ones (defects per level below)
     float c1 = 0.f, c2 = 0.f, c3 = 0.f, c4 = 0.f, br = 0.f, bd = 0.f, be = 0.f;
     if (WEQ == SOFI_EL_ISO || WEQ == SOFI_VEL_ISO) {
-        c1 = ld1<ONE>(m.f, c);
-        c2 = ld1<ONE>(m.g, c);
-        c3 = ld1<ONE>(m.fipjp, c);
+        c1 = ld1<NT>(m.f, c);
+        c2 = ld1<NT>(m.g, c);
+        c3 = ld1<NT>(m.fipjp, c);
     }
     if (WEQ == SOFI_VEL_ISO) {
-        br = ld1<ONE>(m.br, c);
-        bd = ld1<ONE>(m.bd, c);
-        be = ld1<ONE>(m.be, c);
+        br = ld1<NT>(m.br, c);
+        bd = ld1<NT>(m.bd, c);
+        be = ld1<NT>(m.be, c);
     }
     if (WEQ == SOFI_EL_VTI) {
         c1 = m.c11[c];
@@ -1193,9 +1196,9 @@ __device__ __forceinline__ void stress_tile(const Grid &g, const Fields &f0, con
         }
         float vxx, vyx, vxy, vyy;
         if (!stress_dv(g, f, m, fr, i, j, a, b, d, e, vxx, vyx, vxy, vyy)) continue;
-        float sxx = ld1<ONE>(f.sxx, c), syy = ld1<ONE>(f.syy, c),
-              sxy = ld1<ONE>(f.sxy, c);
-        if (WEQ == SOFI_EL_ISO) upd_el(c1, c2, c3, vxx, vyx, vxy, vyy, sxx, syy, sxy, fz, f, g.dt, c);
+        float sxx = ld1<NT>(f.sxx, c), syy = ld1<NT>(f.syy, c),
+              sxy = ld1<NT>(f.sxy, c);
+        if (WEQ == SOFI_EL_ISO) upd_el(g.fma, c1, c2, c3, vxx, vyx, vxy, vyy, sxx, syy, sxy, fz, f, g.dt, c);
         if (WEQ == SOFI_EL_VTI) upd_el_vti(c1, c2, c3, c4, vxx, vyx, vxy, vyy, sxx, syy, sxy, fz, f, g.dt, c);
         if (WEQ == SOFI_VEL_ISO) {
             const float sxyv = vxy + vyx, sdiag = vxx + vyy;
@@ -1204,12 +1207,12 @@ __device__ __forceinline__ void stress_tile(const Grid &g, const Fields &f0, con
             for (int l = 1; l <= SOFI_MAXL; ++l) {
                 if (l > g.L) break;
                 const int o = (l - 1) * g.plane + c;
-                float r = ld1<ONE>(f.r, o), p = ld1<ONE>(f.p, o),
-                      q = ld1<ONE>(f.q, o);
+                float r = ld1<NT>(f.r, o), p = ld1<NT>(f.p, o),
+                      q = ld1<NT>(f.q, o);
                 visc_level(m.eta[l], m.bip[l], m.cip[l], br, bd, be, sxyv, sdiag, vxx, vyy, r, p, q, u);
-                st1<ONE>(f.r, o, r);
-                st1<ONE>(f.p, o, p);
-                st1<ONE>(f.q, o, q);
+                st1<NT>(f.r, o, r);
+                st1<NT>(f.p, o, p);
+                st1<NT>(f.q, o, q);
             }
             visc_final(g.dthalbe, c1, c2, c3, sxyv, sdiag, vxx, vyy, u, sxx, syy, sxy, fz, f, g.dt, c);
         }
@@ -1229,17 +1232,29 @@ __device__ __forceinline__ void stress_tile(const Grid &g, const Fields &f0, con
             visc_vti_final(g.dthalbe, c1, c2, c3, c4, sxyv, vxx, vyy, u, sxx, syy, sxy, fz, f, g.dt, c);
         }
         stress_post<ND, VISCO>(g, f, m, s, fz, fr, nt, i, j, c, sxx, syy, sxy);
-        st1<ONE>(f.sxx, c, sxx);
-        st1<ONE>(f.syy, c, syy);
-        st1<ONE>(f.sxy, c, sxy);
+        st1<NT>(f.sxx, c, sxx);
+        st1<NT>(f.syy, c, syy);
+        st1<NT>(f.sxy, c, sxy);
     }
 }
-template <int ND, int WEQ, bool ONE>
+template <int ND, int WEQ, bool ONE, bool NT = ONE>
 __global__ __launch_bounds__(BX *BY) void k_stress(Grid g, Fields f0, Mat m, Src s, Fuse fz, int nt)
 {
     if (ONE && fused_seis(g, f0, fz)) return;
+    if (ONE) {
+        // in pairs of the two tiles that one tile of k_velocity_r covers: block
+        // 16 q + x and 16 q + 8 + x, which the same XCD gets that had block 8 q +
+        // x of the velocity launch and has its cells in its L2 (us per step
+        // without and with: VEL_ISO FD4 L = 1 613 x 389 10.7 and 10.0, EL_ISO FD4
+        // 400 x 400 10.2 and 9.4)
+        const int b = blockIdx.x, v = (b >> 4) * 8 + (b & 7);
+        if (v >= g.nvtile) return;
+        const int2 t = tile_of(g, 1, 0, v);
+        stress_tile<ND, WEQ, ONE, NT>(g, f0, m, s, fz, nt, t.x, VROWS * t.y + ((b >> 3) & 1));
+        return;
+    }
     const int2 t = tile_of(g, 0, 0, blockIdx.x);
-    stress_tile<ND, WEQ, ONE>(g, f0, m, s, fz, nt, t.x, t.y);
+    stress_tile<ND, WEQ, ONE, NT>(g, f0, m, s, fz, nt, t.x, t.y);
 }
 
 // VW cells per thread (see k_velocity_v); inactive cells (past NX, or
@@ -1316,7 +1331,7 @@ __device__ __forceinline__ void stress_v_slot(const Grid &g, Fields f, const Mat
                 c3 = PRE ? pre[2] : ldv<VW>(m.fipjp, c0);
 #pragma unroll
         for (int k = 0; k < VW; ++k)
-            if (act[k]) upd_el(c1[k], c2[k], c3[k], vxx[k], vyx[k], vxy[k], vyy[k], sxx[k], syy[k], sxy[k], fz, f, g.dt, c0 + k);
+            if (act[k]) upd_el(true, c1[k], c2[k], c3[k], vxx[k], vyx[k], vxy[k], vyy[k], sxx[k], syy[k], sxy[k], fz, f, g.dt, c0 + k);
     }
     if (WEQ == SOFI_EL_VTI) {
         const V c1 = PRE ? pre[0] : ldv<VW>(m.c11, c0), c2 = PRE ? pre[1] : ldv<VW>(m.c13, c0),
@@ -1749,7 +1764,7 @@ __global__ __launch_bounds__(BX *TBY) void k_stress_w(const Shot *__restrict__ s
         const int last = min(ty0 + rows, (d.g.ny + TBY - 1) / TBY);
         for (int ty = ty0; ty < last; ++ty) {
             if constexpr (WEQ == SOFI_AC_ISO) stress_ac_tile<ND, true, TBY>(d.g, d.f, d.m, d.s, d.fs, it, tx, ty);
-            else stress_tile<ND, WEQ, true, TBY>(d.g, d.f, d.m, d.s, d.fs, it, tx, ty);
+            else stress_tile<ND, WEQ, true, true, TBY>(d.g, d.f, d.m, d.s, d.fs, it, tx, ty);
         }
     }
 }
@@ -2078,7 +2093,7 @@ __global__ __launch_bounds__(BX *BY) void k_stress_b(Grid g, Fields f0, Mat m, i
         float vxx, vyx, vxy, vyy;
         if (!stress_dv(g, f, m, fr[q], i, j, a[q], b[q], d[q], e[q], vxx, vyx, vxy, vyy)) continue;
         float sx = sxx[q], sy = syy[q], sz = sxy[q];
-        if (WEQ == SOFI_EL_ISO) upd_el(c1, c2, c3, vxx, vyx, vxy, vyy, sx, sy, sz, fz, f, g.dt, c);
+        if (WEQ == SOFI_EL_ISO) upd_el(false, c1, c2, c3, vxx, vyx, vxy, vyy, sx, sy, sz, fz, f, g.dt, c);
         if (WEQ == SOFI_EL_VTI) upd_el_vti(c1, c2, c3, c4, vxx, vyx, vxy, vyy, sx, sy, sz, fz, f, g.dt, c);
         if (WEQ == SOFI_VEL_ISO) {
             const float sxyv = vxy + vyx, sdiag = vxx + vyy;
@@ -2150,8 +2165,8 @@ __global__ __launch_bounds__(BX *BY) void k_stress_tti_f(Grid g, Fields f0, Mat 
     Park(*const park)[S] = reinterpret_cast<Park(*)[S]>(parks());
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
     __shared__ float sd[S][4][LY][LX];   // dvxx, dvyy, dvyx, dvxy of rows j0-1..j0+BY, columns i0-1..i0+BX
-    // (tiles in plain order: the frame's rows first made one EL_TTI shot 1 % slower)
-    const int ty = div_by(g.tdiv[0], blockIdx.x), tx = blockIdx.x - ty * g.ntx;
+    const int2 t = tile_of(g, 0, 0, blockIdx.x);
+    const int tx = t.x, ty = t.y;
     const int i0 = 1 + tx * BX, j0 = 1 + ty * BY;
     const int k0 = g.k_lo + blockIdx.y * S;
     const bool cpml = g.abs_type == 1 && g.fw > 0;
@@ -2942,6 +2957,8 @@ int sofi_open_batch(const sofi_desc *desc, int nshots, sofi_dev **out)
         g.low[k].first = std::min(d.gy[3], d.ny - 1) / rows;
         g.low[k].n = (d.ny + rows - 1) / rows - g.low[k].first;
     }
+    g.nvtile = g.ntx * ((d.ny + VROWS * BY - 1) / (VROWS * BY));
+    if (d.weq == SOFI_EL_TTI || d.weq == SOFI_VEL_TTI) g.low[0].n = 0;
     for (int k = 0; k < 3; ++k) g.tdiv[k] = fast_div((d.nx + (BX << k) - 1) / (BX << k));
     g.periodic = d.boundary == 1;
     frame_tiles(g);
@@ -3520,19 +3537,47 @@ namespace {
 
 // cells per thread of an ISO/VTI update kernel of the given shape (1: CELL,
 // 2: VEC2, 4: VEC4)
-int vec_width(const Grid &g, int shape)
+int vec_width(int shape)
 {
-    if (shape == SOFI_LAUNCH_CELL) return 1;
     if (shape == SOFI_LAUNCH_VEC2) return 2;
     if (shape == SOFI_LAUNCH_VEC4) return 4;
-    // automatic, as measured on MI355X: the elastic stress updates stream
-    // only 11-12 arrays, too few bytes in flight at one float per thread, and
-    // VEC2 for both kernels won by 26 % (EL_ISO and EL_VTI, 2000 x 1000 FD6:
-    // 48.4 vs 38.5 GLUPS); the viscoelastic ones stream 20-40 arrays and one
-    // cell per thread won (VEL_ISO L=3, 4000 x 2000 FD8: the vector shapes
-    // need 80-150 VGPRs and lose more to occupancy than they gain)
-    return (g.weq == SOFI_EL_ISO || g.weq == SOFI_EL_VTI) ? 2 : 1;
+    // automatic: one cell per thread.  With plain accesses, tiles of both
+    // kernels on the same XCD and the frame's data fetched early it is the
+    // fastest shape at nearly every size (GLUPS, CELL / VEC2 / VEC4: EL_ISO FD8
+    // 1500 x 500 41.2 / 34.2 / 35.9, 2000 x 1000 60.0 / 51.8 / 55.9, 2741 x 1313
+    // 66.3 / 61.1 / 61.8, 4000 x 2000 67.5 / 47.0 / 56.9; EL_VTI FD6 2000 x 1000
+    // 59.5 / 59.0 / 58.9, 3000 x 1700 70.1 / 75.8 / 69.1, 4000 x 2000 68.8 / 52.5
+    // / 61.4; VEL_ISO L = 3 FD8 1000 x 1000 30.1 / 28.5 / 25.9, 2000 x 1000 37.4 /
+    // 36.2 / 35.8, 4000 x 2000 37.5 / 27.1 / 28.8)
+    return 1;
 }
+
+// Bytes that a step of the slots' handle goes through: the wavefields of the
+// slots and the medium arrays its updates read.
+size_t step_bytes(const Grid &g, int slots)
+{
+    size_t medium = 2;                                       // rip, rjp
+    switch (g.weq) {
+      case SOFI_AC_ISO: medium += 1; break;
+      case SOFI_EL_ISO: medium += 3; break;
+      case SOFI_VEL_ISO: medium += 6; break;
+      case SOFI_EL_VTI: medium += 4; break;
+      case SOFI_VEL_VTI: medium += 4 + 4 * (size_t)g.L; break;
+      default: medium += 8 * (size_t)(1 + g.L);
+    }
+    return ((5 + 3 * (size_t)g.L) * (size_t)slots + medium) * (size_t)g.plane * sizeof(float);
+}
+
+// Above this much the one-slot kernels use nontemporal hints (see k_velocity):
+// a step's data no longer stays in the 256 MB memory-side cache from one step
+// to the next, and what streams past leaves room for the stencil rows.  Below,
+// the hints keep out of the cache what the next kernel wants there.  GLUPS
+// with plain accesses / hints: EL_ISO FD8 2000 x 1000 (79 MiB) 60.0 / 50.5, 3000
+// x 1700 (201 MiB) 72.6 / 62.1, 4000 x 2000 (310 MiB) 65.8 / 67.5; VEL_ISO FD8 L
+// = 1 2741 x 1313 (228 MiB) 51.3 / 45.8, 3000 x 1700 (322 MiB) 49.3 / 49.2; L = 3
+// 1000 x 1000 (87 MiB) 30.1 / 23.7, 2741 x 1313 (314 MiB) 32.9 / 32.4, 3000 x
+// 1700 (442 MiB) 33.2 / 35.4, 4000 x 2000 (682 MiB) 32.9 / 36.5.
+constexpr size_t NT_BYTES = (size_t)300 << 20;
 
 // One time step.  With ntb set the step is captured into a block: nt is the
 // block's local step (1..K), the kernels add the base step held at ntb, and
@@ -3831,6 +3876,7 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
     if (te) (void)hipEventRecord(te[0], st);
     for (int lo = lo0; lo < hi0; lo += grp) {
         Grid gg = g;
+        gg.fma = h->shape_s == SOFI_LAUNCH_AUTO;
         gg.k_lo = lo;
         gg.k_hi = lo + grp < hi0 ? lo + grp : hi0;
         const int nchunk = (gg.k_hi - lo + g.spt - 1) / g.spt;   // groups of g.spt slots (blockIdx.y)
@@ -3907,6 +3953,7 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
             continue;
         }
         // a launch of one slot runs the one-shot kernels on that slot's fields
+        const bool nt_hints = step_bytes(g, span) > NT_BYTES;
         const bool one = gg.k_hi - gg.k_lo == 1;
         const Fields fk = one ? f.at(lo, g) : f;
         Fuse fv_l = fv;
@@ -3916,7 +3963,7 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
             fv_l.soff = sf.soff;
             fv_l.nforce = sf.nforce;
         }
-        int vw = vec_width(g, h->shape_v);
+        int vw = vec_width(h->shape_v);
         dim3 tiles((g.nx + BX * vw - 1) / (BX * vw) * nty, nchunk);
         const dim3 vtiles((unsigned)(g.ntx * ((g.ny + VROWS * BY - 1) / (VROWS * BY))));   // one slot, VROWS rows per thread
         if (h->wl) {
@@ -3935,11 +3982,13 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
         else if (vw == 2 && one) launch_lds(h, k_velocity_v<ND, 2, true>, tiles, blk, park_bytes(g, 2), gg, fk, m, h->s, fv_l, nt);
         else if (vw == 2) launch_lds(h, k_velocity_v<ND, 2, false>, tiles, blk, park_bytes(g, 2), gg, fk, m, h->s, fv_l, nt);
         else if (one && tti) launch_lds(h, k_velocity<ND, true, false>, tiles, blk, park_bytes(g, 1), gg, fk, m, h->s, fv_l, nt);
+        else if (one && !nt_hints) launch_lds(h, k_velocity_r<ND, false, VROWS>, vtiles, blk, park_bytes(g, VROWS), gg, fk, m, h->s, fv_l, nt);
         else if (one) launch_lds(h, k_velocity_r<ND, true, VROWS>, vtiles, blk, park_bytes(g, VROWS), gg, fk, m, h->s, fv_l, nt);
         else launch_lds(h, k_velocity<ND, false>, tiles, blk, park_bytes(g, 1), gg, fk, m, h->s, fv_l, nt);
         wrap_x(h, gg, lo, gg.k_hi, f.vx, f.vy);
-        vw = vec_width(g, h->shape_s);
+        vw = vec_width(h->shape_s);
         tiles = dim3((g.nx + BX * vw - 1) / (BX * vw) * nty, nchunk);
+        if (vw == 1 && one && d.weq != SOFI_AC_ISO && !tti) tiles = dim3((unsigned)((g.nvtile + 7) / 8 * 16));
         // vx / vy sampling in extra blocks of a one-slot stress launch
         Fuse fss = fs;
         if (slot_fused) {
@@ -3966,6 +4015,7 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
             else if (vw == 4) launch_lds(h, k_stress_v<ND, W, 4, false>, tiles, blk, park_bytes(g, 4), gg, fk, m, h->s, fss, nt);    \
             else if (vw == 2 && one) launch_lds(h, k_stress_v<ND, W, 2, true>, tiles, blk, park_bytes(g, 2), gg, fk, m, h->s, fss, nt);   \
             else if (vw == 2) launch_lds(h, k_stress_v<ND, W, 2, false>, tiles, blk, park_bytes(g, 2), gg, fk, m, h->s, fss, nt);    \
+            else if (one && !nt_hints) launch_lds(h, k_stress<ND, W, true, false>, tiles, blk, park_bytes(g, 1), gg, fk, m, h->s, fss, nt); \
             else if (one) launch_lds(h, k_stress<ND, W, true>, tiles, blk, park_bytes(g, 1), gg, fk, m, h->s, fss, nt);              \
             else launch_lds(h, k_stress<ND, W, false>, tiles, blk, park_bytes(g, 1), gg, fk, m, h->s, fss, nt);            \
         } while (0)

@@ -273,8 +273,8 @@ int sofi_fwi_residual_noalloc(sofi_dev *h, const sofi_residual_opts *opts, const
  * cell in 64 x 4 tiles, SOFI_LAUNCH_VEC2 / SOFI_LAUNCH_VEC4 one thread per
  * two / four consecutive cells of a row (vector loads and stores) in
  * 128 x 4 / 256 x 4 tiles, SOFI_LAUNCH_AUTO (the default) the shape
- * measured fastest for the rheology (VEC2 for EL_ISO / EL_VTI, CELL
- * otherwise), for one-shot handles and batches alike.  Results agree to
+ * measured fastest (CELL, for EL_ISO with VEC2's rounding of the stress
+ * update), for one-shot handles and batches alike.  Results agree to
  * rounding between shapes and bit for bit between a batch slot and a
  * one-shot handle of the same shape. */
 enum { SOFI_LAUNCH_AUTO = 0, SOFI_LAUNCH_CELL = 1, SOFI_LAUNCH_VEC2 = 2, SOFI_LAUNCH_VEC4 = 3 };
