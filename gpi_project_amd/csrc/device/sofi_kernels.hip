@@ -325,7 +325,7 @@ __device__ __forceinline__ float div_k(const Grid &g, const Mat &m, float x, int
 // CPML on the stress-side derivatives of one frame cell (cpml_update_s_x/_y,
 // src/cpml_update.c:30-46); updates the psi memory and returns modified values.
 __device__ __forceinline__ void cpml_dv(const Grid &g, const Mat &m, Fields &f, const Frame &o, int i, int j,
-                                        float &vxx, float &vyx, float &vxy, float &vyy)
+                                        float &vxx, float &vyx, float &vxy, float &vyy, const float4v *pre = nullptr)
 {
     const int lane = threadIdx.x;
     frame_wait();
@@ -343,7 +343,7 @@ __device__ __forceinline__ void cpml_dv(const Grid &g, const Mat &m, Fields &f, 
     if (o.yf) {
         const int h = hy(g, __builtin_amdgcn_readfirstlane(j));
         const int q = h * g.wy + i;
-        const auto cy = m.pmly[h];
+        const auto cy = pre ? *pre : m.pmly[h];         // pre: fetched before
         const float py = __builtin_fmaf(cy[0], o.pk->y0[lane], cy[1] * vyy);
         f.psi_vyy[q] = py;
         vyy = div_k(g, m, vyy, SOFI_P_K_Y, h) + py;
@@ -566,19 +566,25 @@ enum { SURF_T1 = 0, SURF_T2, SURF_G, SURF_DE, SURF_FG, SURF_N };
 // variables) with the horizontal derivative only; in the x-CPML the second
 // update of psi_vxx[1][h] in the same step is reproduced.  sxx is the cell's
 // value after the stress update and source injection; returns the new one.
-template <int ND, bool VISCO>
-__device__ __forceinline__ float surface_sxx(const Grid &g, Fields &f, const Mat &m, int i, int c, float sxx)
+// vxx, vyy: the cell's raw sums of op_s (no 1/DH).
+struct SurfC {
+    float t1, t2, gg, de, fg;
+};
+template <bool VISCO>
+__device__ __forceinline__ SurfC surface_coef(const Grid &g, const Mat &m, int i)
 {
-    const int j = 1, P = g.pitch;
+    const float *sc = m.surf + (i - 1);
+    return { sc[SURF_T1 * g.nx], sc[SURF_T2 * g.nx], sc[SURF_G * g.nx], VISCO ? sc[SURF_DE * g.nx] : 0.f,
+             VISCO ? sc[SURF_FG * g.nx] : 0.f };
+}
+template <bool VISCO>
+__device__ __forceinline__ float surface_fix(const Grid &g, Fields &f, const Mat &m, const SurfC &sc, int i, int c,
+                                             float sxx, float vxx, float vyy)
+{
+    const int j = 1;
     const float dhi = (float)(1.0 / g.dh);
     if (VISCO)
         for (int l = 1; l <= g.L; ++l) f.q[(l - 1) * g.plane + c] = 0.0f;
-    float vxx = 0.f, vyy = 0.f;
-#pragma unroll
-    for (int m1 = 1; m1 <= ND; ++m1) {
-        vxx += g.hc[m1] * (f.vx[c + m1 - 1] - f.vx[c - m1]);
-        vyy += g.hc[m1] * (f.vy[c + (m1 - 1) * P] - f.vy[c - m1 * P]);
-    }
     vxx *= dhi;
     vyy *= dhi;
     if (g.abs_type == 1 && !g.periodic) {   // no x-CPML at a periodic edge (src/surface_elastic.c:64-78)
@@ -595,15 +601,14 @@ __device__ __forceinline__ float surface_sxx(const Grid &g, Fields &f, const Mat
             vxx = vxx / PRF(g, m, SOFI_P_K_X, h) + ps;
         }
     }
-    const float *sc = m.surf + (i - 1);
-    const float t1 = sc[SURF_T1 * g.nx], t2 = sc[SURF_T2 * g.nx], gg = sc[SURF_G * g.nx];
+    const float t1 = sc.t1, t2 = sc.t2, gg = sc.gg;
     if (!VISCO) {
         sxx += -(t1 * vxx / gg) - (t2 * vyy);
     } else {
         float sump = 0.f;
         for (int l = 1; l <= g.L; ++l) sump += f.p[(l - 1) * g.plane + c];
         sxx += -(t1 * vxx / gg) - (t2 * vyy) - (g.dthalbe * sump);
-        const float de = sc[SURF_DE * g.nx], fg = sc[SURF_FG * g.nx];
+        const float de = sc.de, fg = sc.fg;
         sump = 0.f;
         for (int l = 1; l <= g.L; ++l) {
             float &pv = f.p[(l - 1) * g.plane + c];
@@ -613,6 +618,19 @@ __device__ __forceinline__ float surface_sxx(const Grid &g, Fields &f, const Mat
         sxx += (g.dthalbe * sump);
     }
     return sxx;
+}
+
+template <int ND, bool VISCO>
+__device__ __forceinline__ float surface_sxx(const Grid &g, Fields &f, const Mat &m, int i, int c, float sxx)
+{
+    const int P = g.pitch;
+    float vxx = 0.f, vyy = 0.f;
+#pragma unroll
+    for (int m1 = 1; m1 <= ND; ++m1) {
+        vxx += g.hc[m1] * (f.vx[c + m1 - 1] - f.vx[c - m1]);
+        vyy += g.hc[m1] * (f.vy[c + (m1 - 1) * P] - f.vy[c - m1 * P]);
+    }
+    return surface_fix<VISCO>(g, f, m, surface_coef<VISCO>(g, m, i), i, c, sxx, vxx, vyy);
 }
 
 // the free surface as a pass of its own, after the stress update and sources
@@ -633,6 +651,13 @@ __global__ void k_surface(Grid g, Fields f0, Mat m)
 }
 
 // ------------------------------------------------------------ tile mapping
+
+// of n tiles, the q-th of XCD x (0..7) when each gets a contiguous share: one
+// to one over 8 q + x < n
+__device__ __forceinline__ int xcd_band(int x, int q, int n)
+{
+    return x * (n >> 3) + min(x, n & 7) + q;
+}
 
 // Tiles of the ISO/VTI update kernels are numbered row-major over the grid
 // in workgroup order.  The hardware hands workgroups round-robin to the
@@ -846,10 +871,10 @@ __global__ __launch_bounds__(BX *BY) void k_velocity_r(Grid g, Fields f, Mat m, 
 {
     Park(*const park)[R] = reinterpret_cast<Park(*)[R]>(parks());
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    static_assert(R == VROWS, "tile_of's rows");
     const int2 t = tile_of(g, 1, 0, blockIdx.x);
     const int tx = t.x, ty = t.y;
     const int i = 1 + tx * BX + threadIdx.x;
-    static_assert(R == VROWS, "tile_of's rows");
     const int j = 1 + ty * R * BY + R * threadIdx.y;
     if (i > g.nx || j > g.ny) return;
     const int nr = min(R, g.ny - j + 1);
@@ -1011,14 +1036,17 @@ __device__ __forceinline__ void upd_el(bool one, float f_, float g_, float fipjp
     fwi_u_store(fz, f, dt, c, u1, u2, u3);
 }
 
-// wavefield_update_s_el_vti (src/wavefield_update_s_el_vti.c:27-47)
+// wavefield_update_s_el_vti (src/wavefield_update_s_el_vti.c:27-47).  Which
+// products are fused is written out: left to the compiler it depends on the
+// blocks around the update, and every kernel has to round alike.
 __device__ __forceinline__ void upd_el_vti(float c11, float c13, float c33, float c55i, float vxx, float vyx,
                                            float vxy, float vyy, float &sxx, float &syy, float &sxy, const Fuse &fz,
                                            const Fields &f, float dt, int c)
 {
+#pragma clang fp contract(off)
     const float u1 = c55i * (vxy + vyx);
-    const float u2 = (c11 * vxx) + (c13 * vyy);
-    const float u3 = (c13 * vxx) + (c33 * vyy);
+    const float u2 = __builtin_fmaf(c11, vxx, c13 * vyy);
+    const float u3 = __builtin_fmaf(c13, vxx, c33 * vyy);
     sxy += u1;
     sxx += u2;
     syy += u3;
@@ -1096,7 +1124,7 @@ __device__ __forceinline__ void visc_vti_final(float dthalbe, float u11, float u
 // reference never updates (ABS_TYPE other than 1 or 2).
 __device__ __forceinline__ bool stress_dv(const Grid &g, Fields &f, const Mat &m, const Frame &fr, int i, int j,
                                           float a, float b, float d, float e, float &vxx, float &vyx, float &vxy,
-                                          float &vyy)
+                                          float &vyy, const float4v *cy = nullptr)
 {
     const bool frame = fr.any();
     if (frame && g.abs_type != 1 && g.abs_type != 2) return false;
@@ -1104,7 +1132,7 @@ __device__ __forceinline__ bool stress_dv(const Grid &g, Fields &f, const Mat &m
     vyx = b * g.dhi;
     vxy = d * g.dhi;
     vyy = e * g.dhi;
-    if (g.abs_type == 1 && frame) cpml_dv(g, m, f, fr, i, j, vxx, vyx, vxy, vyy);
+    if (g.abs_type == 1 && frame) cpml_dv(g, m, f, fr, i, j, vxx, vyx, vxy, vyy, cy);
     return true;
 }
 
@@ -1113,9 +1141,19 @@ __device__ __forceinline__ bool stress_dv(const Grid &g, Fields &f, const Mat &m
 // to the same cell when it is fused here: the explosive sources (psource) and
 // the free surface (imaging into the ghost rows by the cells that are imaged,
 // correction of row 1).
-template <int ND, bool VISCO>
+// EARLY: what the caller has fetched or computed before: the amplitude of the
+// first explosive source in the cell, the free surface's coefficients and the
+// raw velocity sums of the cell.
+struct Early {
+    int k = -1;                 // the source, and its amplitude
+    float amp = 0.f;
+    SurfC sc{};
+    float vxx = 0.f, vyy = 0.f;
+};
+template <int ND, bool VISCO, bool EARLY = false>
 __device__ __forceinline__ void stress_post(const Grid &g, Fields &f, const Mat &m, const Src &s, const Fuse &fz,
-                                            const Frame &fr, int nt, int i, int j, int c, float &sxx, float &syy, float &sxy)
+                                            const Frame &fr, int nt, int i, int j, int c, float &sxx, float &syy, float &sxy,
+                                            const Early &pre = {})
 {
     if (g.abs_type == 2 && fr.any()) {
         const float q = m.absorb[c];
@@ -1125,7 +1163,7 @@ __device__ __forceinline__ void stress_post(const Grid &g, Fields &f, const Mat 
     }
     for (int k = 0; k < fz.npsrc; ++k)
         if (c == fz.c[k]) {
-            const float amp = psource_amp(g, s, fz.soff + k, step_of(fz.ntb, nt));
+            const float amp = EARLY && k == pre.k ? pre.amp : psource_amp(g, s, fz.soff + k, step_of(fz.ntb, nt));
             sxx += amp;
             syy += amp;
         }
@@ -1135,7 +1173,8 @@ __device__ __forceinline__ void stress_post(const Grid &g, Fields &f, const Mat 
         if (j <= ND) f.sxy[c + (1 - 2 * j) * P] = -sxy;  // sxy(1 - m) = -sxy(m)
         if (j == 1) {
             syy = 0.0f;
-            sxx = surface_sxx<ND, VISCO>(g, f, m, i, c, sxx);
+            sxx = EARLY ? surface_fix<VISCO>(g, f, m, pre.sc, i, c, sxx, pre.vxx, pre.vyy)
+                        : surface_sxx<ND, VISCO>(g, f, m, i, c, sxx);
         }
     }
 }
@@ -1255,6 +1294,263 @@ __global__ __launch_bounds__(BX *BY) void k_stress(Grid g, Fields f0, Mat m, Src
     }
     const int2 t = tile_of(g, 0, 0, blockIdx.x);
     stress_tile<ND, WEQ, ONE, NT>(g, f0, m, s, fz, nt, t.x, t.y);
+}
+
+// ------------------------------------------------- a whole step in one launch
+
+// What the one-launch step writes instead of updating in place: neighbouring
+// blocks still read the old values.  The two sets of a handle change places
+// after each step.
+struct Next {
+    float *vx, *vy, *sxx, *syy, *sxy;
+    float *psi_sxx_x, *psi_sxy_x, *psi_syy_y, *psi_sxy_y;
+};
+
+// velocities of cell (i, j) after the step; the same operations in the same
+// order as op_v and velocity_core.  OWN: a cell of the block's own tile, whose
+// CPML memory and FWI planes the block writes; else one of the ring around it.
+template <int ND, bool OWN>
+__device__ __forceinline__ void step_velocity(const Grid &g, const Fields &f, const Next &n, const Mat &m, const Src &s,
+                                              const Fuse &fz, int nt, int i, int j, int c, float &vx, float &vy,
+                                              float4v &cy)
+{
+    const bool xf = in_xframe(g, i), yf = in_yframe(g, j);
+    const bool pml = g.abs_type == 1 && (xf || yf);
+    float x0 = 0.f, x1 = 0.f, y0 = 0.f, y1 = 0.f;
+    float4v cx = {};
+    int h = 0, qx = 0, qy = 0, k = 0;
+    if (pml && xf) {
+        h = hx(g, i);
+        qx = j * g.wx + h;
+        cx = m.pmlx[h];
+        x0 = f.psi_sxx_x[qx];
+        x1 = f.psi_sxy_x[qx];
+    }
+    if (pml && yf) {
+        k = hy(g, j);
+        qy = k * g.wy + i;
+        cy = m.pmly[k];
+        y0 = f.psi_syy_y[qy];
+        y1 = f.psi_sxy_y[qy];
+    }
+    const float rip = m.rip[c], rjp = m.rjp[c];
+    vx = f.vx[c];
+    vy = f.vy[c];
+    float sxx_x, sxy_x, sxy_y, syy_y;
+    op_v<ND>(g, f.sxx, f.syy, f.sxy, c, sxx_x, sxy_x, sxy_y, syy_y);
+    if (OWN && i == g.nx / 2 && j == g.ny / 2 && isnan(vy) && *f.unstable == 0) *f.unstable = step_of(fz.ntb, nt);
+    if (pml && xf) {
+        const float a = __builtin_fmaf(cx[2], x0, cx[3] * sxx_x);
+        sxx_x = div_k(g, m, sxx_x, SOFI_P_K_X_HALF, h) + a;
+        const float b = __builtin_fmaf(cx[0], x1, cx[1] * sxy_x);
+        sxy_x = div_k(g, m, sxy_x, SOFI_P_K_X, h) + b;
+        if (OWN) {
+            n.psi_sxx_x[qx] = a;
+            n.psi_sxy_x[qx] = b;
+        }
+    }
+    if (pml && yf) {
+        const float a = __builtin_fmaf(cy[2], y0, cy[3] * syy_y);
+        syy_y = div_k(g, m, syy_y, SOFI_P_K_Y_HALF, k) + a;
+        const float b = __builtin_fmaf(cy[0], y1, cy[1] * sxy_y);
+        sxy_y = div_k(g, m, sxy_y, SOFI_P_K_Y, k) + b;
+        if (OWN) {
+            n.psi_syy_y[qy] = a;
+            n.psi_sxy_y[qy] = b;
+        }
+    }
+    for (int q = 0; q < fz.nforce; ++q)
+        if (c == fz.c[q]) force_add(g, s, fz.soff + q, step_of(fz.ntb, nt), rip, rjp, vx, vy);
+    if (OWN) {
+        if (fz.fwi_acc == 1) {
+            f.pvxp1[c] = rip * (sxx_x + sxy_y) / g.dh;
+            f.pvyp1[c] = rjp * (sxy_x + syy_y) / g.dh;
+        } else if (fz.fwi_acc == 2) {
+            f.pvxp1[c] += vx * g.dt;
+            f.pvyp1[c] += vy * g.dt;
+        } else if (fz.fwi_acc == 3) {
+            f.pvxp1[c] = vx;
+            f.pvyp1[c] = vy;
+        }
+    }
+    vx = vx + (sxx_x + sxy_y) * g.dtdh * rip;
+    vy = vy + (sxy_x + syy_y) * g.dtdh * rjp;
+    if (g.abs_type == 2 && (xf || yf)) {
+        const float a = m.absorb[c];
+        vx *= a;
+        vy *= a;
+    }
+}
+
+// rows of a block's tile (a wave each) and waves for the ring of ND cells
+// around it, one cell per lane for orders up to 8
+template <int ND>
+struct StepTile {
+    static constexpr int RING = 2 * ND * BX;
+    static constexpr int TY = ND == 4 ? 7 : 8;
+    static constexpr int W0 = (RING + 2 * ND * TY + BX - 1) / BX;
+    static constexpr int EW = W0 < 16 - TY ? W0 : 16 - TY;
+};
+
+// A grid of up to ONE_LAUNCH_CELLS cells is bound by the trips of a launch to
+// memory and by the gap between launches, not by bandwidth: the velocity and
+// the stress kernel took 4.4 us each for 97 x 83 cells as for 300 x 300.  Here
+// a block computes the new velocities of its tile and of a ring of ND cells
+// around it into LDS, from the old fields, and updates the tile's stresses
+// from there: one launch, one chain of trips.  The tile's waves fetch what
+// their stress update needs before the barrier; the ring has waves of its own,
+// beside and not after the tile's.  Tiles in bands of the XCDs (xcd_band): the
+// rings of most tiles are then in the L2 that the step before wrote them to
+// (EL_ISO FD4 400 x 400 8.4 us per step, in plain order 10.1; tiles of 4 rows
+// 8.9, of 11 rows 9.1).  us per step of the two kernels (in the same bands) and
+// of this one: EL_ISO FD4 97 x 83 8.9 and 7.1, 300 x 300 8.9 and 7.1; VEL_ISO L
+// = 3 FD8 300 x 300 11.1 and 8.8.  (VEL_VTI, whose defects cannot all be fetched
+// early, gained 2 to 7 %, and not with the same rounding: two kernels.)
+// Above, the ring's work costs more than the second launch: EL_ISO FD8 400 x
+// 400 10.3 and 10.7, 700 x 700 13.9 and 20.2.
+template <int ND, int WEQ>
+__global__ __launch_bounds__(BX *(StepTile<ND>::TY + StepTile<ND>::EW)) void k_step(Grid g, Fields f0, Next n, Mat m,
+                                                                                  Src s, Fuse fv, Fuse fs, int nt, int ntile, int seismo)
+{
+    using T = StepTile<ND>;
+    constexpr int TY = T::TY, W = BX + 2 * ND;
+    constexpr bool VISCO = WEQ == SOFI_VEL_ISO;
+    __shared__ float lx[TY + 2 * ND][W], ly[TY + 2 * ND][W];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.y), lane = threadIdx.x;
+    if (fs.sblk && (int)blockIdx.x >= fs.ntile) {
+        // receivers of the step before, whose fields this launch reads
+        const int k = ((int)blockIdx.x - fs.ntile) * (BX * (TY + T::EW)) + w * BX + lane;
+        if (k < fs.rec.n) seis_sample(g, f0, fs.rec, k, fs.ntb ? (fs.ins + *fs.ntb) / fs.ndt : fs.ins, seismo);
+        return;
+    }
+    const int tile = xcd_band(blockIdx.x & 7, blockIdx.x >> 3, ntile);
+    const int ty = div_by(g.tdiv[0], tile), tx = tile - ty * g.tdiv[0].d;
+    const int i0 = 1 + tx * BX, j0 = 1 + ty * TY;
+    const int i = i0 + lane, j = j0 + w, c = IDX(g, i, j), P = g.pitch;
+    const bool own = w < TY && i <= g.nx && j <= g.ny;
+    Park *const park = parks();
+    Frame fr;
+    float c1 = 0.f, c2 = 0.f, c3 = 0.f, c4 = 0.f, br = 0.f, bd = 0.f, be = 0.f, sxx = 0.f, syy = 0.f, sxy = 0.f;
+    float r[SOFI_MAXL], p[SOFI_MAXL], q[SOFI_MAXL];
+    float4v cy = {};
+    Early pre;
+    if (w >= TY) {
+        for (int t = (w - TY) * BX + lane; t < T::RING + 2 * ND * TY; t += T::EW * BX) {
+            int li, lj;
+            if (t < T::RING) {
+                lj = t / BX;
+                lj = lj < ND ? lj : lj + TY;
+                li = ND + (t & (BX - 1));
+            } else {
+                const int e = t - T::RING;
+                lj = e / (2 * ND);
+                li = e - lj * (2 * ND);
+                li = li < ND ? li : li + BX;
+                lj += ND;
+            }
+            const int ii = i0 - ND + li, jj = j0 - ND + lj, cc = IDX(g, ii, jj);
+            float vx = 0.f, vy = 0.f;
+            float4v cy = {};
+            if (ii >= 1 && ii <= g.nx && jj >= 1 && jj <= g.ny) {
+                step_velocity<ND, false>(g, f0, n, m, s, fv, nt, ii, jj, cc, vx, vy, cy);
+            } else if (ii <= g.nx + ND && jj <= g.ny + ND) {
+                vx = f0.vx[cc];             // the padding around the grid
+                vy = f0.vy[cc];
+            }
+            lx[lj][li] = vx;
+            ly[lj][li] = vy;
+        }
+    } else {
+        float vx = 0.f, vy = 0.f;
+        if (own) {
+            fr = frame_load<false>(g, f0, m, i, j, c, park[w]);
+            if (WEQ == SOFI_EL_ISO || WEQ == SOFI_VEL_ISO) {
+                c1 = m.f[c];
+                c2 = m.g[c];
+                c3 = m.fipjp[c];
+            }
+            if (WEQ == SOFI_VEL_ISO) {
+                br = m.br[c];
+                bd = m.bd[c];
+                be = m.be[c];
+            }
+            if (WEQ == SOFI_EL_VTI) {
+                c1 = m.c11[c];
+                c2 = m.c13[c];
+                c3 = m.c33[c];
+                c4 = m.c55i[c];
+            }
+            sxx = f0.sxx[c];
+            syy = f0.syy[c];
+            sxy = f0.sxy[c];
+            if (VISCO) {
+#pragma unroll
+                for (int l = 0; l < SOFI_MAXL; ++l) {
+                    if (l >= g.L) break;
+                    r[l] = f0.r[l * g.plane + c];
+                    p[l] = f0.p[l * g.plane + c];
+                    q[l] = f0.q[l * g.plane + c];
+                }
+            }
+            for (int k = fs.npsrc - 1; k >= 0; --k)
+                if (c == fs.c[k]) {
+                    pre.k = k;
+                    pre.amp = psource_amp(g, s, fs.soff + k, step_of(fs.ntb, nt));
+                }
+            if (fs.surf && j == 1) pre.sc = surface_coef<VISCO>(g, m, i);
+            step_velocity<ND, true>(g, f0, n, m, s, fv, nt, i, j, c, vx, vy, cy);
+            n.vx[c] = vx;
+            n.vy[c] = vy;
+        } else if (i <= g.nx + ND && j <= g.ny + ND) {
+            vx = f0.vx[c];
+            vy = f0.vy[c];
+        }
+        lx[w + ND][lane + ND] = vx;
+        ly[w + ND][lane + ND] = vy;
+    }
+    __syncthreads();
+    if (!own) return;
+    Fields f = f0;
+    f.vx = n.vx;
+    f.vy = n.vy;
+    f.sxx = n.sxx;
+    f.syy = n.syy;
+    f.sxy = n.sxy;
+    const int li = lane + ND, lj = w + ND;
+    float a = 0.f, b = 0.f, d = 0.f, e = 0.f;
+#pragma unroll
+    for (int mm = 1; mm <= ND; ++mm) {
+        const float h = g.hc[mm];
+        a += h * (lx[lj][li + mm - 1] - lx[lj][li - mm]);
+        b += h * (ly[lj][li + mm] - ly[lj][li - mm + 1]);
+        d += h * (lx[lj + mm][li] - lx[lj - mm + 1][li]);
+        e += h * (ly[lj + mm - 1][li] - ly[lj - mm][li]);
+    }
+    float vxx, vyx, vxy, vyy;
+    stress_dv(g, f, m, fr, i, j, a, b, d, e, vxx, vyx, vxy, vyy, &cy);
+    if (WEQ == SOFI_EL_ISO) upd_el(g.fma, c1, c2, c3, vxx, vyx, vxy, vyy, sxx, syy, sxy, fs, f, g.dt, c);
+    if (WEQ == SOFI_EL_VTI) upd_el_vti(c1, c2, c3, c4, vxx, vyx, vxy, vyy, sxx, syy, sxy, fs, f, g.dt, c);
+    if (VISCO) {
+        const float sxyv = vxy + vyx, sdiag = vxx + vyy;
+        VSum u;
+#pragma unroll
+        for (int l = 1; l <= SOFI_MAXL; ++l) {
+            if (l > g.L) break;
+            const int o = (l - 1) * g.plane + c;
+            float rl = r[l - 1], pl = p[l - 1], ql = q[l - 1];
+            visc_level(m.eta[l], m.bip[l], m.cip[l], br, bd, be, sxyv, sdiag, vxx, vyy, rl, pl, ql, u);
+            f.r[o] = rl;
+            f.p[o] = pl;
+            f.q[o] = ql;
+        }
+        visc_final(g.dthalbe, c1, c2, c3, sxyv, sdiag, vxx, vyy, u, sxx, syy, sxy, fs, f, g.dt, c);
+    }
+    pre.vxx = a;
+    pre.vyy = e;
+    stress_post<ND, VISCO, true>(g, f, m, s, fs, fr, nt, i, j, c, sxx, syy, sxy, pre);
+    f.sxx[c] = sxx;
+    f.syy[c] = syy;
+    f.sxy[c] = sxy;
 }
 
 // VW cells per thread (see k_velocity_v); inactive cells (past NX, or
@@ -2714,6 +3010,9 @@ struct sofi_dev {
     std::vector<NodeArgs> gargs;
     hipError_t gerr = hipSuccess;
     int graph_k = 0;
+    Next alt{};                            // the second set of the one-launch step (none: vx is null)
+    bool one_launch = false;               // while a block is recorded: its steps are one launch each
+    int pend = 0;                          // and the local step whose receivers the next launch samples (0: none)
     unsigned gen = 1, graph_gen = 0;       // launch configuration: current / of the captured graph
     long long graph_blocks = 0;            // blocks replayed since the handle opened
     // a batch's resident groups: res_mode slots (0: chosen from the cache
@@ -2771,6 +3070,17 @@ void frame_tiles(Grid &g)
     if (g.ftop + g.fbot > g.nty) g.fbot = g.nty - g.ftop;
     if (g.fl > g.ntx) g.fl = g.ntx;
     if (g.fl + g.fr > g.ntx) g.fr = g.ntx - g.fl;
+}
+
+// Handles whose captured blocks may run one launch per step: see k_step for
+// both sides of the line
+constexpr size_t ONE_LAUNCH_CELLS = size_t(1) << 17;
+bool one_launch_fits(const sofi_dev *h)
+{
+    const sofi_desc &d = h->d;
+    return h->nb == 1 && d.fdorder_time != 4 && (d.weq == SOFI_EL_ISO || d.weq == SOFI_VEL_ISO || d.weq == SOFI_EL_VTI) &&
+           d.boundary != 1 && (d.fw == 0 || d.abs_type == 1 || d.abs_type == 2) &&
+           d.seismo != 3 && d.seismo != 4 && (size_t)d.nx * d.ny <= ONE_LAUNCH_CELLS;
 }
 
 int dalloc(sofi_dev *h, void **p, size_t bytes)
@@ -3034,6 +3344,14 @@ int sofi_open_batch(const sofi_desc *desc, int nshots, sofi_dev **out)
         rc |= dalloc_t(h, &f.psi_sxy_y, nyp);
         rc |= dalloc_t(h, &f.psi_vyy, nyp);
         rc |= dalloc_t(h, &f.psi_vxy, nyp);
+    }
+    if (one_launch_fits(h)) {
+        Next &n = h->alt;
+        for (float **q : { &n.vx, &n.vy, &n.sxx, &n.syy, &n.sxy }) rc |= dalloc_t(h, q, pl);
+        if (f.psi_sxx_x) {
+            for (float **q : { &n.psi_sxx_x, &n.psi_sxy_x }) rc |= dalloc_t(h, q, (size_t)g.nxp);
+            for (float **q : { &n.psi_syy_y, &n.psi_sxy_y }) rc |= dalloc_t(h, q, (size_t)g.nyp);
+        }
     }
     if (d.mode == SOFI_MODE_FWI) {
         if (d.weq == SOFI_AC_ISO) {
@@ -3864,6 +4182,41 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
     if (adj && h->nadj > 0)
         launch(h, k_adjoint, dim3((h->adj_inj.n + 63) / 64), dim3(64), g, f, h->adj_inj, h->adj_sx,
                            h->adj_sy, d.nt, d.adjoint_type, nt, ntb);
+    // a whole step in one launch; vx / vy / p of step nt are sampled by the next
+    // step's launch, or after the block's last (not where forces of a launch of
+    // their own change the velocities before that)
+    bool seis_late = false;
+    if (h->one_launch) {
+        Grid gg = g;
+        gg.fma = h->shape_s == SOFI_LAUNCH_AUTO;
+        seis_late = sample && !(nsrc > 0 && h->any_force && !fv.nforce);
+        Fuse fss = fs;
+        using T = StepTile<ND>;
+        const int ntile = g.ntx * ((g.ny + T::TY - 1) / T::TY);
+        dim3 tiles((unsigned)ntile), tb(BX, T::TY + T::EW);
+        if (h->pend) {
+            fss.ntile = ntile;
+            fss.sblk = (rr.n + BX * (int)tb.y - 1) / (BX * (int)tb.y);
+            fss.ins = h->pend;
+            fss.ndt = ndt;
+            fss.rec = rr;
+            tiles.x += fss.sblk;
+        }
+        h->pend = seis_late ? ins : 0;
+        auto *k = d.weq == SOFI_EL_ISO ? k_step<ND, SOFI_EL_ISO> : d.weq == SOFI_VEL_ISO ? k_step<ND, SOFI_VEL_ISO>
+                                             : k_step<ND, SOFI_EL_VTI>;
+        launch_lds(h, k, tiles, tb, park_bytes(g, 1, T::TY), gg, f, h->alt, m, h->s, fv, fss, nt, ntile, d.seismo);
+        Next &n = h->alt;
+        std::swap(f.vx, n.vx);
+        std::swap(f.vy, n.vy);
+        std::swap(f.sxx, n.sxx);
+        std::swap(f.syy, n.syy);
+        std::swap(f.sxy, n.sxy);
+        std::swap(f.psi_sxx_x, n.psi_sxx_x);
+        std::swap(f.psi_sxy_x, n.psi_sxy_x);
+        std::swap(f.psi_syy_y, n.psi_syy_y);
+        std::swap(f.psi_sxy_y, n.psi_sxy_y);
+    }
     hipEvent_t *te = nullptr;
     if (!inblk && !h->wl && h->time_every > 0 && nt % h->time_every == 0 && h->tev_used + 4 <= (int)h->tev.size()) {
         te = &h->tev[h->tev_used];
@@ -3874,7 +4227,7 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
     // the update kernels, launched per group of h->grp slots (all slots of a
     // one-shot handle or of an untuned batch: one group)
     if (te) (void)hipEventRecord(te[0], st);
-    for (int lo = lo0; lo < hi0; lo += grp) {
+    for (int lo = lo0; lo < hi0 && !h->one_launch; lo += grp) {
         Grid gg = g;
         gg.fma = h->shape_s == SOFI_LAUNCH_AUTO;
         gg.k_lo = lo;
@@ -3965,7 +4318,7 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
         }
         int vw = vec_width(h->shape_v);
         dim3 tiles((g.nx + BX * vw - 1) / (BX * vw) * nty, nchunk);
-        const dim3 vtiles((unsigned)(g.ntx * ((g.ny + VROWS * BY - 1) / (VROWS * BY))));   // one slot, VROWS rows per thread
+        const dim3 vtiles((unsigned)g.nvtile);   // one slot, VROWS rows per thread
         if (h->wl) {
             // the work-list launch of sofi_run_many covers this update
             h->wl_shot.g = gg;
@@ -4085,7 +4438,7 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
     wrap_x(h, g, lo0, hi0, d.weq == SOFI_AC_ISO ? nullptr : f.sxy, f.sxx);
     if (sample && d.seismo != 3 && h->wl) {
         h->wl_seis = ins;
-    } else if (sample && d.seismo != 3 && !seis_fused) {
+    } else if (sample && d.seismo != 3 && !(h->one_launch ? seis_late : seis_fused)) {
         dim3 rb(64), rg((rr.n + 63) / 64);
         launch(h, k_seis, rg, rb, g, f, rr, ins, d.seismo, ntb, ndt);
     }
@@ -4124,6 +4477,13 @@ int step(sofi_dev *h, int nt, const int *ntb = nullptr)
     return fail("unsupported ND %d", h->g.nd);
 }
 
+// captured blocks of an even number of steps, so that the two sets of the
+// wavefields have changed back at a block's end, run one launch per step
+bool one_launch(const sofi_dev *h)
+{
+    return h->alt.vx && h->shape_v == SOFI_LAUNCH_AUTO && h->shape_s == SOFI_LAUNCH_AUTO;
+}
+
 constexpr size_t GRAPH_AUTO_CELLS = size_t(1) << 20;
 constexpr int GRAPH_STEPS = 64;
 
@@ -4143,7 +4503,8 @@ int graph_len(const sofi_dev *h)
         unit = unit / a * dtinv;
     }
     const int want = h->graph_steps > 0 ? h->graph_steps : GRAPH_STEPS;
-    return (want + unit - 1) / unit * unit;
+    const int k = (want + unit - 1) / unit * unit;
+    return one_launch(h) && h->graph_steps <= 0 && k % 2 ? k + unit : k;
 }
 
 // a block of k steps may start at nt when it ends before nt_last and the
@@ -4187,7 +4548,17 @@ int run_block(sofi_dev *h, int nt, int k)
         h->glast = nullptr;
         h->gerr = hipSuccess;
         int rc = 0;
+        const Fields f0 = h->f;
+        const Next n0 = h->alt;
+        h->one_launch = k % 2 == 0 && one_launch(h);
+        h->pend = 0;
         for (int l = 1; l <= k && !rc; ++l) rc = step(h, l, h->ntb);
+        if (h->pend && !rc)
+            launch(h, k_seis, dim3((h->r.n + 63) / 64), dim3(64), h->g, h->f, h->r, h->pend, h->d.seismo, h->ntb,
+                   h->d.ndt > 0 ? h->d.ndt : 1);
+        h->one_launch = false;
+        h->f = f0;
+        h->alt = n0;
         h->gbuild = nullptr;
         const hipError_t e = h->gerr;
         h->gerr = hipSuccess;
