@@ -86,6 +86,7 @@ struct Grid {
     // tile rows of the lower absorbing frame, in tiles of BY and of VROWS BY rows
     struct { int first, n; } low[2];
     int nvtile;         // tiles of VROWS BY rows
+    bool band;          // each XCD has a contiguous band of the tiles (see BAND_BYTES)
     bool fma;           // EL_ISO: see upd_el
     int wx, wy;     // row lengths of x-frame and y-frame CPML memory
     int ntx;        // tiles along x of the one-cell-per-thread update kernels
@@ -671,9 +672,15 @@ __device__ __forceinline__ int xcd_band(int x, int q, int n)
 // longer than the others, and a launch that ends with them ends late (EL_ISO
 // FD8 with CPML, us per step with and without: 1500 x 500 20.1 and 21.1, 2000 x
 // 1000 38.8 and 39.1, 2741 x 1313 59.2 and 59.7).
+// That order is for data that streams from HBM; below BAND_BYTES each XCD has a
+// band of its own (Grid::band), in which no tile row comes first.
 // Block b's tile: 2^vw cells per thread in x, rows in y as of g.low[k].
 __device__ __forceinline__ int2 tile_of(const Grid &g, int k, int vw, int b)
 {
+    if (g.band) {
+        const int t = xcd_band(b & 7, b >> 3, k ? g.nvtile : g.tdiv[vw].d * g.nty), r = div_by(g.tdiv[vw], t);
+        return make_int2(t - r * g.tdiv[vw].d, r);
+    }
     const int r = div_by(g.tdiv[vw], b), n = g.low[k].n;
     return make_int2(b - r * g.tdiv[vw].d, r < n ? g.low[k].first + r : r - n);
 }
@@ -3072,6 +3079,24 @@ void frame_tiles(Grid &g)
     if (g.fl + g.fr > g.ntx) g.fr = g.ntx - g.fl;
 }
 
+size_t step_bytes(const Grid &g, int slots);
+
+// A shot's step up to this much runs with its tiles in bands of the XCDs
+// (tile_of): its data stays in the 256 MB memory-side cache, and what a tile
+// shares with its neighbours and with the step before is found in the XCD's
+// own L2.  Above, the bands read eight places of HBM at once and lose.  us per
+// step in plain order and in bands: EL_ISO FD4 400 x 400 10.8 and 9.6, 700 x
+// 700 15.2 and 12.2, 1400 x 1400 35.4 and 30.3; EL_ISO FD8 2000 x 1000 50.2 and
+// 45.0, 3400 x 1700 (220 MiB) 124 and 108; VEL_ISO L = 3 2000 x 1000 (174 MB)
+// 68.6 and 63.0; L = 1 2741 x 1313 (228 MB) 92.7 and 85.9, 3400 x 1700 (352 MiB)
+// 152.5 and 154.3; L = 3 2741 x 1313 (314 MiB) 131 and 143, 4000 x 2000 270 and
+// 283; batches of 2000 x 1000, EL_VTI 8 shots 224 and 210, EL_TTI 4 shots 196
+// and 178.  TTI: the top and bottom frame tiles, with the most work, fall to
+// one XCD each, which a small grid feels: 2000 x 1000 59.5 and 55.3, VEL_TTI 803
+// x 607 32.9 and 34.0.
+constexpr size_t BAND_BYTES = (size_t)256 << 20;
+constexpr size_t BAND_TTI_CELLS = (size_t)1 << 19;
+
 // Handles whose captured blocks may run one launch per step: see k_step for
 // both sides of the line
 constexpr size_t ONE_LAUNCH_CELLS = size_t(1) << 17;
@@ -3268,6 +3293,8 @@ int sofi_open_batch(const sofi_desc *desc, int nshots, sofi_dev **out)
         g.low[k].n = (d.ny + rows - 1) / rows - g.low[k].first;
     }
     g.nvtile = g.ntx * ((d.ny + VROWS * BY - 1) / (VROWS * BY));
+    const bool tti = d.weq == SOFI_EL_TTI || d.weq == SOFI_VEL_TTI;
+    g.band = step_bytes(g, 1) <= BAND_BYTES && (!tti || (size_t)d.nx * d.ny >= BAND_TTI_CELLS);
     if (d.weq == SOFI_EL_TTI || d.weq == SOFI_VEL_TTI) g.low[0].n = 0;
     for (int k = 0; k < 3; ++k) g.tdiv[k] = fast_div((d.nx + (BX << k) - 1) / (BX << k));
     g.periodic = d.boundary == 1;
