@@ -283,7 +283,8 @@ int sofi_set_launch(sofi_dev *h, int velocity_shape, int stress_shape);
 /* Captured blocks of time steps.  The reference's time loop launches every
  * step's updates one after the other (src/time_loop.c:40-325); here sofi_run
  * records `steps` consecutive steps (rounded up to a multiple of NDT, and of
- * DTINV for FWI; 0: 64) once into a HIP graph whose kernels read the block's
+ * DTINV for FWI; 0: 64, rounded up to an even number for small grids, whose
+ * even blocks run one launch per step) once into a HIP graph whose kernels read the block's
  * base step from device memory, and replays it for every block that starts
  * on a sampling (and FWI store) boundary and holds no snapshot and not the
  * loop's last step; the other steps run one by one.  SOFI_GRAPH_AUTO (the
