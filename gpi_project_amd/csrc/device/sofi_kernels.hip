@@ -33,6 +33,7 @@
 
 #include "sofi_hip.h"
 #include "../common/sofi_iir.h"
+#include "sofi_frame.h"
 
 namespace {
 
@@ -193,11 +194,6 @@ __device__ __forceinline__ int IDX(const Grid &g, int i, int j) { return (j - 1 
 // CPML profile k (enum sofi_profile) at index h
 __device__ __forceinline__ float PRF(const Grid &g, const Mat &m, int k, int h) { return m.prof[k * (2 * g.fw + 1) + h]; }
 
-__device__ __forceinline__ bool in_xframe(const Grid &g, int i) { return i <= g.gx2 || i > g.gx3; }
-__device__ __forceinline__ bool in_yframe(const Grid &g, int j) { return j <= g.gy2 || j > g.gy3; }
-__device__ __forceinline__ int hx(const Grid &g, int i) { return i <= g.gx2 ? i : i - g.nx + 2 * g.fw; }
-__device__ __forceinline__ int hy(const Grid &g, int j) { return j <= g.gy2 ? j : j - g.ny + 2 * g.fw; }
-
 // ------------------------------------------------------------ FD stencils
 
 // op_v_fd* (src/initfd.c:97-183): stress derivatives, no 1/DH
@@ -285,23 +281,23 @@ __device__ __forceinline__ void to_lds(const float4v *src, float4v *dst)
 }
 
 // V: for the velocity update, else the stress update; one wave per tile row
-// (j is the same in all its lanes), lane = threadIdx.x
-template <bool V>
+// (j is the same in all its lanes), lane = threadIdx.x.  PAST: see sofi_frame.h
+template <bool V, bool PAST = false>
 __device__ __forceinline__ Frame frame_load(const Grid &g, const Fields &f, const Mat &m, int i, int j, int c, Park &pk)
 {
     const int ju = __builtin_amdgcn_readfirstlane(j);
     Frame o;
-    o.xf = in_xframe(g, i);
-    o.yf = in_yframe(g, ju);
+    o.xf = frame_x<PAST>(g, i);
+    o.yf = frame_y<PAST>(g, i, ju);
     o.pk = &pk;
-    if (g.abs_type == 1) {
+    if (cpml_fetch<PAST>(g)) {
         if (o.yf) {
-            const int q = hy(g, ju) * g.wy + i;
+            const int q = y_entry(g, i, ju);
             to_lds((V ? f.psi_syy_y : f.psi_vyy) + q, pk.y0);
             to_lds((V ? f.psi_sxy_y : f.psi_vxy) + q, pk.y1);
         }
         if (o.xf) {
-            const int h = hx(g, i), q = ju * g.wx + h;
+            const int h = hx(g, i), q = x_entry(g, h, ju);
             to_lds(m.pmlx + h, pk.cx);
             to_lds((V ? f.psi_sxx_x : f.psi_vxx) + q, pk.x0);
             to_lds((V ? f.psi_sxy_x : f.psi_vyx) + q, pk.x1);
@@ -950,9 +946,9 @@ __device__ __forceinline__ void velocity_v_slot(const Grid &g, Fields f, const M
     }
     V vx = ldv<VW>(f.vx, c0), vy = ldv<VW>(f.vy, c0);
     const V rip = PRE ? pre[0] : ldv<VW>(m.rip, c0), rjp = PRE ? pre[1] : ldv<VW>(m.rjp, c0);
-    Frame fr[VW];      // (a cell past NX fetches the neighbouring entries, which nothing uses)
+    Frame fr[VW];      // (nothing for a cell past NX)
 #pragma unroll
-    for (int k = 0; k < VW; ++k) fr[k] = frame_load<true>(g, f, m, i0 + k, j, c0 + k, park[k]);
+    for (int k = 0; k < VW; ++k) fr[k] = frame_load<true, true>(g, f, m, i0 + k, j, c0 + k, park[k]);
     float d[VW] = {}, e[VW] = {};
 #pragma unroll
     for (int mm = 1; mm <= ND; ++mm) {
@@ -1592,9 +1588,9 @@ __device__ __forceinline__ void stress_v_slot(const Grid &g, Fields f, const Mat
         }
         b0[mm - 1] = ldv<VW>(f.vy, c0 - mm * P);
     }
-    Frame fr[VW];      // (a cell past NX fetches the neighbouring entries, which nothing uses)
+    Frame fr[VW];      // (nothing for a cell past NX)
 #pragma unroll
-    for (int k = 0; k < VW; ++k) fr[k] = frame_load<false>(g, f, m, i0 + k, j, c0 + k, park[k]);
+    for (int k = 0; k < VW; ++k) fr[k] = frame_load<false, true>(g, f, m, i0 + k, j, c0 + k, park[k]);
     float d[VW] = {}, e[VW] = {};
 #pragma unroll
     for (int mm = 1; mm <= ND; ++mm) {
