@@ -2286,8 +2286,12 @@ __global__ void k_wrap_x(Grid g, float *a, float *b)
 // sampling run as separate launches; the per-cell arithmetic of a slot is
 // that of the one-thread-per-cell kernels.
 
+// FD order 12 with one slot per thread is held to 64 registers, so that 8 waves
+// fit a SIMD: the frame fetch had taken it to 66, and six EL_ISO shots of 1008 x
+// 707 with a damping frame from 61.9 to 63.2 us per step (61.9 again; with CPML
+// 66.6 and 65.8).  The other kernels of one slot per thread need 56 or fewer.
 template <int ND, int S>
-__global__ __launch_bounds__(BX *BY) void k_velocity_b(Grid g, Fields f0, Mat m, int nt, const int *ntb, int fwi_acc)
+__global__ __launch_bounds__(BX *BY, ND == 6 && S == 1 ? 8 : 1) void k_velocity_b(Grid g, Fields f0, Mat m, int nt, const int *ntb, int fwi_acc)
 {
     Park(*const park)[S] = reinterpret_cast<Park(*)[S]>(parks());
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
