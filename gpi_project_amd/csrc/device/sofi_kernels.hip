@@ -87,7 +87,7 @@ struct Grid {
     // tile rows of the lower absorbing frame, in tiles of BY and of VROWS BY rows
     struct { int first, n; } low[2];
     int nvtile;         // tiles of VROWS BY rows
-    bool band;          // each XCD has a contiguous band of the tiles (see BAND_BYTES)
+    int band;           // 1: each XCD has a contiguous band of the tiles (see BAND_BYTES), 0: plain order
     bool fma;           // EL_ISO: see upd_el
     int wx, wy;     // row lengths of x-frame and y-frame CPML memory
     int ntx;        // tiles along x of the one-cell-per-thread update kernels
@@ -681,6 +681,15 @@ __device__ __forceinline__ int2 tile_of(const Grid &g, int k, int vw, int b)
     return make_int2(b - r * g.tdiv[vw].d, r < n ? g.low[k].first + r : r - n);
 }
 
+// The same where no row comes first: the TTI kernels.  One piece of code, so
+// that its arguments are loaded together: each branch of tile_of is a trip to
+// memory of its own before a tile's first load.
+__device__ __forceinline__ int2 tile_in_order(const Grid &g, int b)
+{
+    const int t = b + (-g.band & (xcd_band(b & 7, b >> 3, g.ntx * g.nty) - b)), r = div_by(g.tdiv[0], t);
+    return make_int2(t - r * g.ntx, r);
+}
+
 // Tile shapes: CELL, one thread per cell in BX x BY tiles (also the TTI
 // passes); VEC2 / VEC4, one thread per VW = 2 / 4 consecutive cells of a row
 // in (VW BX) x BY tiles, every stencil row and coefficient fetched as one
@@ -855,7 +864,7 @@ __device__ __forceinline__ void velocity_tile(const Grid &g, const Fields &f0, c
 template <int ND, bool ONE, bool NT = ONE>
 __global__ __launch_bounds__(BX *BY) void k_velocity(Grid g, Fields f0, Mat m, Src s, Fuse fz, int nt)
 {
-    const int2 t = tile_of(g, 0, 0, blockIdx.x);
+    const int2 t = ONE ? tile_in_order(g, blockIdx.x) : tile_of(g, 0, 0, blockIdx.x);     // one slot: TTI only
     velocity_tile<ND, ONE, NT>(g, f0, m, s, fz, nt, t.x, t.y);
 }
 
@@ -2460,20 +2469,19 @@ __global__ __launch_bounds__(BX *BY) void k_stress_b(Grid g, Fields f0, Mat m, i
 //     pass to follow) are added to their cells after the update, as psource
 //     does after the stress update (src/time_loop.c:248-250).
 // S slots per thread (blockIdx.y: group of S slots of a batch; 1 for a
-// one-shot handle).
-template <int ND, int WEQ, int S>
+// one-shot handle).  PML: the grid may have a CPML frame (see tti_update).
+template <int ND, int WEQ, int S, bool PML>
 __global__ __launch_bounds__(BX *BY) void k_stress_tti_f(Grid g, Fields f0, Mat m, Fuse fz, Src src, int nt)
 {
     constexpr int LX = BX + 2, LY = BY + 2;
     Park(*const park)[S] = reinterpret_cast<Park(*)[S]>(parks());
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
     __shared__ float sd[S][4][LY][LX];   // dvxx, dvyy, dvyx, dvxy of rows j0-1..j0+BY, columns i0-1..i0+BX
-    const int2 t = tile_of(g, 0, 0, blockIdx.x);
+    const int2 t = tile_in_order(g, blockIdx.x);
     const int tx = t.x, ty = t.y;
     const int i0 = 1 + tx * BX, j0 = 1 + ty * BY;
     const int k0 = g.k_lo + blockIdx.y * S;
-    const bool cpml = g.abs_type == 1 && g.fw > 0;
-    const bool store_dv = cpml && is_frame_tile(g, tx, ty);
+    const bool store_dv = PML && g.abs_type == 1 && g.fw > 0 && is_frame_tile(g, tx, ty);
     const int tid = threadIdx.y * BX + threadIdx.x;
     const int i = i0 + threadIdx.x, j = j0 + threadIdx.y;
     Frame fr[S];
@@ -4103,13 +4111,32 @@ struct StrB {
         static auto fn() { return k_stress_b<ND, WEQ, S>; }
     };
 };
-template <int ND, int WEQ>
+template <int ND, int WEQ, bool PML>
 struct TtiF {
     template <int S>
     struct K {
-        static auto fn() { return k_stress_tti_f<ND, WEQ, S>; }
+        static auto fn() { return k_stress_tti_f<ND, WEQ, S, PML>; }
     };
 };
+
+// k_stress_tti_f of slots lo..hi-1, S per thread.  Without a CPML frame the
+// kernel that knows of none: the frame's code takes scalar registers from every
+// wave, so that arguments are loaded one after the other and spilled (EL_TTI FD8
+// with a damping frame, us per step with that code and without: 400 x 1000 19.2
+// and 17.2, 700 x 700 21.3 and 19.7, 2000 x 1000 43.1 and 40.8; VEL_TTI FD8 1500
+// x 900 37.7 and 36.2).  From FD8 on, above what the memory-side cache holds, the
+// kernel with that code is the faster one (EL_TTI FD8 4000 x 2000 185.6 and 190.0,
+// FD12 3000 x 1500 120 and 123; but FD6 4000 x 2000 176 and 170); both hold 8
+// waves per SIMD at FD8, and why it is faster there is not known.
+template <int ND>
+void tti_update(sofi_dev *h, const Grid &gg, int lo, int hi, int S, const Fields &f, const Mat &m, const Fuse &fz, int nt)
+{
+    const bool pml = (gg.abs_type == 1 && gg.fw > 0) || (ND > 3 && step_bytes(gg, 1) > BAND_BYTES);
+    if (gg.weq == SOFI_EL_TTI && pml) launch_blocks<ND, TtiF<ND, SOFI_EL_TTI, true>::template K>(h, gg, lo, hi, S, f, m, fz, h->s, nt);
+    else if (gg.weq == SOFI_EL_TTI) launch_blocks<ND, TtiF<ND, SOFI_EL_TTI, false>::template K>(h, gg, lo, hi, S, f, m, fz, h->s, nt);
+    else if (pml) launch_blocks<ND, TtiF<ND, SOFI_VEL_TTI, true>::template K>(h, gg, lo, hi, S, f, m, fz, h->s, nt);
+    else launch_blocks<ND, TtiF<ND, SOFI_VEL_TTI, false>::template K>(h, gg, lo, hi, S, f, m, fz, h->s, nt);
+}
 
 template <int ND>
 int step_nd(sofi_dev *h, int nt, const int *ntb)
@@ -4325,8 +4352,7 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
                   }
                   Fuse fin = f0;
                   if (g.abs_type == 1 && g.fw > 0 && frame_tile_count(g) > 0) fin.npsrc = 0;
-                  if (d.weq == SOFI_EL_TTI) launch_blocks<ND, TtiF<ND, SOFI_EL_TTI>::template K>(h, gg, lo, gg.k_hi, S, f, m, fin, h->s, nt);
-                  else launch_blocks<ND, TtiF<ND, SOFI_VEL_TTI>::template K>(h, gg, lo, gg.k_hi, S, f, m, fin, h->s, nt);
+                  tti_update<ND>(h, gg, lo, gg.k_hi, S, f, m, fin, nt);
                   tti_frame<ND>(h, gg, lo, gg.k_hi, f, m, f0, nt);
               }
             }
@@ -4428,8 +4454,7 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
               const bool frame_passes = g.abs_type == 1 && g.fw > 0 && frame_tile_count(g) > 0;
               Fuse fin = fss;
               if (frame_passes) fin.npsrc = 0;
-              if (d.weq == SOFI_EL_TTI) launch_blocks<ND, TtiF<ND, SOFI_EL_TTI>::template K>(h, gg, lo, gg.k_hi, 1, f, m, fin, h->s, nt);
-              else launch_blocks<ND, TtiF<ND, SOFI_VEL_TTI>::template K>(h, gg, lo, gg.k_hi, 1, f, m, fin, h->s, nt);
+              tti_update<ND>(h, gg, lo, gg.k_hi, 1, f, m, fin, nt);
               tti_frame<ND>(h, gg, lo, gg.k_hi, f, m, fss, nt);
           }
         }
