@@ -681,9 +681,10 @@ __device__ __forceinline__ int2 tile_of(const Grid &g, int k, int vw, int b)
     return make_int2(b - r * g.tdiv[vw].d, r < n ? g.low[k].first + r : r - n);
 }
 
-// The same where no row comes first: the TTI kernels.  One piece of code, so
-// that its arguments are loaded together: each branch of tile_of is a trip to
-// memory of its own before a tile's first load.
+// The same where no row comes first: the TTI kernels, and 4th order in time
+// without CPML.  One piece of code, so that its arguments are loaded together:
+// each branch of tile_of is a trip to memory of its own before a tile's first
+// load.
 __device__ __forceinline__ int2 tile_in_order(const Grid &g, int b)
 {
     const int t = b + (-g.band & (xcd_band(b & 7, b >> 3, g.ntx * g.nty) - b)), r = div_by(g.tdiv[0], t);
@@ -1789,12 +1790,16 @@ struct Hist4 {
 // src/wavefield_update_v_4.c:25-47), one thread per cell.  Forces first; in
 // the CPML frame the left side and the four corners only advance the CPML
 // memory and keep their velocities, as the reference's loops do.
-template <int ND>
+// PML: CPML frame (EL_ISO FD8 with a damping frame, us per step with the CPML
+// code in the kernel and without, 4th order in time: 500 x 500 11.3 and 10.6; VEL_ISO
+// L = 3 400 x 400 14.2 and 13.4)
+template <int ND, bool PML>
 __global__ __launch_bounds__(BX *BY) void k_velocity4(Grid g, Fields f, Mat m, Src s, Fuse fz, int nt, Hist4 H)
 {
+    __builtin_assume(PML == (g.abs_type == 1));
     Park *const park = parks();
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
-    const int2 t = tile_of(g, 0, 0, blockIdx.x);
+    const int2 t = PML ? tile_of(g, 0, 0, blockIdx.x) : tile_in_order(g, blockIdx.x);
     const int tx = t.x, ty = t.y;
     const int i = 1 + tx * BX + threadIdx.x;
     const int j = 1 + ty * BY + threadIdx.y;
@@ -1838,13 +1843,14 @@ __global__ __launch_bounds__(BX *BY) void k_velocity4(Grid g, Fields f, Mat m, S
 // their own histories (written into [3]), the stress update, then damping,
 // the fused sources and the free surface as in the 2nd-order kernel, which
 // see the memory variables just written.
-template <int ND, bool VISCO>
+template <int ND, bool VISCO, bool PML>
 __global__ __launch_bounds__(BX *BY) void k_stress4(Grid g, Fields f, Mat m, Src s, Fuse fz, int nt, Hist4 H)
 {
+    __builtin_assume(PML == (g.abs_type == 1));
     Park *const park = parks();
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
     if (fused_seis(g, f, fz)) return;
-    const int2 t = tile_of(g, 0, 0, blockIdx.x);
+    const int2 t = PML ? tile_of(g, 0, 0, blockIdx.x) : tile_in_order(g, blockIdx.x);
     const int tx = t.x, ty = t.y;
     const int i = 1 + tx * BX + threadIdx.x;
     const int j = 1 + ty * BY + threadIdx.y;
@@ -3087,7 +3093,7 @@ void frame_tiles(Grid &g)
     if (g.fl + g.fr > g.ntx) g.fr = g.ntx - g.fl;
 }
 
-size_t step_bytes(const Grid &g, int slots);
+size_t step_bytes(const Grid &g, int slots, bool fdt4 = false);
 
 // A shot's step up to this much runs with its tiles in bands of the XCDs
 // (tile_of): its data stays in the 256 MB memory-side cache, and what a tile
@@ -3104,6 +3110,14 @@ size_t step_bytes(const Grid &g, int slots);
 // x 607 32.9 and 34.0.
 constexpr size_t BAND_BYTES = (size_t)256 << 20;
 constexpr size_t BAND_TTI_CELLS = (size_t)1 << 19;
+// At 4th order in time, whose histories are most of a step's bytes (step_bytes
+// counts them), bands gain up to here only (us per step, plain order and bands,
+// FD8: EL_ISO 800 x 800, 88 MiB, 23.0 and 20.5; 1200 x 900, 144 MiB, 35.8 and
+// 29.9; 1500 x 900, 182 MiB, 39.9 and 36.5; 1700 x 1000, 228 MiB, 54.6 and 59.0;
+// 3000 x 1500, 604 MiB, 145 and 157; VEL_ISO L = 1 1000 x 800, 156 MiB, 34.0 and
+// 33.7; 1500 x 900, 263 MiB, 62.3 and 65.8.  2000 x 1000 is better in bands, by 1
+// to 2 %: 72.1 and 71.1, L = 3 156.8 and 153.)
+constexpr size_t BAND4_BYTES = (size_t)200 << 20;
 
 // Handles whose captured blocks may run one launch per step: see k_step for
 // both sides of the line
@@ -3302,7 +3316,8 @@ int sofi_open_batch(const sofi_desc *desc, int nshots, sofi_dev **out)
     }
     g.nvtile = g.ntx * ((d.ny + VROWS * BY - 1) / (VROWS * BY));
     const bool tti = d.weq == SOFI_EL_TTI || d.weq == SOFI_VEL_TTI;
-    g.band = step_bytes(g, 1) <= BAND_BYTES && (!tti || (size_t)d.nx * d.ny >= BAND_TTI_CELLS);
+    const bool fdt4 = d.fdorder_time == 4;
+    g.band = step_bytes(g, 1, fdt4) <= (fdt4 ? BAND4_BYTES : BAND_BYTES) && (!tti || (size_t)d.nx * d.ny >= BAND_TTI_CELLS);
     if (d.weq == SOFI_EL_TTI || d.weq == SOFI_VEL_TTI) g.low[0].n = 0;
     for (int k = 0; k < 3; ++k) g.tdiv[k] = fast_div((d.nx + (BX << k) - 1) / (BX << k));
     g.periodic = d.boundary == 1;
@@ -3906,8 +3921,9 @@ int vec_width(int shape)
 }
 
 // Bytes that a step of the slots' handle goes through: the wavefields of the
-// slots and the medium arrays its updates read.
-size_t step_bytes(const Grid &g, int slots)
+// slots (at 4th order in time their histories) and the medium arrays its
+// updates read.
+size_t step_bytes(const Grid &g, int slots, bool fdt4)
 {
     size_t medium = 2;                                       // rip, rjp
     switch (g.weq) {
@@ -3918,7 +3934,8 @@ size_t step_bytes(const Grid &g, int slots)
       case SOFI_VEL_VTI: medium += 4 + 4 * (size_t)g.L; break;
       default: medium += 8 * (size_t)(1 + g.L);
     }
-    return ((5 + 3 * (size_t)g.L) * (size_t)slots + medium) * (size_t)g.plane * sizeof(float);
+    const size_t field = 5 + 3 * (size_t)g.L + (fdt4 ? 24 + 9 * (size_t)g.L : 0);
+    return (field * (size_t)slots + medium) * (size_t)g.plane * sizeof(float);
 }
 
 // Above this much the one-slot kernels use nontemporal hints (see k_velocity):
@@ -4294,7 +4311,8 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
             // update (src/time_loop.c:89-91,226-244); the memory variables
             // the rest of the step sees are the ones just written
             const dim3 t4((g.nx + BX - 1) / BX * nty);
-            launch_lds(h, k_velocity4<ND>, t4, blk, park_bytes(g, 1), gg, f, m, h->s, fv, nt, h->h4);
+            const bool pml = g.abs_type == 1;
+            launch_lds(h, pml ? k_velocity4<ND, true> : k_velocity4<ND, false>, t4, blk, park_bytes(g, 1), gg, f, m, h->s, fv, nt, h->h4);
             wrap_x(h, gg, lo, gg.k_hi, f.vx, f.vy);
             rot4(h->h4.sx);
             rot4(h->h4.sy);
@@ -4312,8 +4330,8 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
                 fss.rec = rr;
                 ts.x += fss.sblk;
             }
-            if (g.L > 0) launch_lds(h, k_stress4<ND, true>, ts, blk, park_bytes(g, 1), gg, f, m, h->s, fss, nt, h->h4);
-            else launch_lds(h, k_stress4<ND, false>, ts, blk, park_bytes(g, 1), gg, f, m, h->s, fss, nt, h->h4);
+            if (g.L > 0) launch_lds(h, pml ? k_stress4<ND, true, true> : k_stress4<ND, true, false>, ts, blk, park_bytes(g, 1), gg, f, m, h->s, fss, nt, h->h4);
+            else launch_lds(h, pml ? k_stress4<ND, false, true> : k_stress4<ND, false, false>, ts, blk, park_bytes(g, 1), gg, f, m, h->s, fss, nt, h->h4);
             for (int q = 0; q < 4; ++q) rot4(h->h4.dv[q]);
             if (g.L > 0) {
                 rot4(h->h4.r);

@@ -1,6 +1,6 @@
-"""The TTI kernels without CPML code and the tile order of both kinds, at the
-sizes where the choice between them changes and with sources in every part of
-the grid.  Whole wavefields against the FP32 oracle,
+"""Kernels without CPML code (TTI rheologies, 4th order in time) and the tile
+orders of both, at the sizes where the choice between them changes and with
+sources in every part of the grid.  Whole wavefields against the FP32 oracle,
 1e-5, the bound of the other parity tests."""
 import os
 import tempfile
@@ -22,6 +22,10 @@ DH, DT = 5.0, 4.0e-4
     ("VEL_TTI", 1, 8, 2, 900, 583, 8),       # and past it
     ("EL_TTI", 0, 8, 2, 2900, 1401, 4),      # 238 MiB per step: both sides of the
     ("EL_TTI", 0, 8, 2, 3001, 1501, 4),      # 267 MiB             memory-side cache
+    ("EL_ISO", 0, 8, 4, 131, 67, 40),
+    ("VEL_ISO", 2, 6, 4, 190, 130, 20),
+    ("EL_ISO", 0, 8, 4, 1500, 961, 8),       # 4th order in time, 194 MiB with its histories: bands
+    ("EL_ISO", 0, 8, 4, 1600, 961, 8),       # and 210 MiB: plain order
 ])
 def test_tiles_match_oracle(weq, L, fdorder, fdt, nx, ny, steps, abs_type):
     import pyoracle
@@ -52,7 +56,8 @@ def test_tiles_match_oracle(weq, L, fdorder, fdt, nx, ny, steps, abs_type):
         for fid in range(5):
             a = sim.field(fid).ravel().astype(np.float64)
             e = rel_l2(a, o.field(fid))
-            assert e <= 1e-5 and np.any(a), (fid, e)
+            # (at 4th order in time the reference sets no shear modulus: sxy stays zero)
+            assert e <= 1e-5 and (np.any(a) or (fid == 4 and fdt == 4)), (fid, e)
         o.close()
         sim.close()
         P.close()
