@@ -3122,10 +3122,9 @@ constexpr size_t BAND4_BYTES = (size_t)200 << 20;
 // Handles whose captured blocks may run one launch per step: see k_step for
 // both sides of the line
 constexpr size_t ONE_LAUNCH_CELLS = size_t(1) << 17;
-bool one_launch_fits(const sofi_dev *h)
+bool one_launch_fits(const sofi_desc &d, int nshots)
 {
-    const sofi_desc &d = h->d;
-    return h->nb == 1 && d.fdorder_time != 4 && (d.weq == SOFI_EL_ISO || d.weq == SOFI_VEL_ISO || d.weq == SOFI_EL_VTI) &&
+    return nshots == 1 && d.fdorder_time != 4 && (d.weq == SOFI_EL_ISO || d.weq == SOFI_VEL_ISO || d.weq == SOFI_EL_VTI) &&
            d.boundary != 1 && (d.fw == 0 || d.abs_type == 1 || d.abs_type == 2) &&
            d.seismo != 3 && d.seismo != 4 && (size_t)d.nx * d.ny <= ONE_LAUNCH_CELLS;
 }
@@ -3395,7 +3394,7 @@ int sofi_open_batch(const sofi_desc *desc, int nshots, sofi_dev **out)
         rc |= dalloc_t(h, &f.psi_vyy, nyp);
         rc |= dalloc_t(h, &f.psi_vxy, nyp);
     }
-    if (one_launch_fits(h)) {
+    if (one_launch_fits(d, nshots)) {
         Next &n = h->alt;
         for (float **q : { &n.vx, &n.vy, &n.sxx, &n.syy, &n.sxy }) rc |= dalloc_t(h, q, pl);
         if (f.psi_sxx_x) {
@@ -5701,8 +5700,13 @@ size_t sofi_estimate_footprint(const sofi_desc *d, int nshots, int ntr, int nsna
         b += 24 * (pl + A);
         if (visco) b += 9 * (pl * L + A);
     }
-    if (d->abs_type == 1 && d->fw > 0)
-        b += 4 * ((size_t)(d->ny + 1) * wx * 4 * nb + A) + 4 * (wx * (size_t)(d->nx + 1) * 4 * nb + A);
+    // CPML memory, and the second set of the one-launch step: velocities,
+    // stresses and the velocity update's CPML memory
+    const size_t mx = (size_t)(d->ny + 1) * wx * 4 * nb + A, my = wx * (size_t)(d->nx + 1) * 4 * nb + A;
+    const bool cpml = d->abs_type == 1 && d->fw > 0, second = one_launch_fits(*d, nshots);
+    if (cpml) b += 4 * mx + 4 * my;
+    if (second) b += 5 * (pl + A);
+    if (second && cpml) b += 2 * mx + 2 * my;
     size_t arrays = 4;                                                        // rip rjp pu ppi
     switch (d->weq) {
       case SOFI_EL_ISO: arrays += 3; break;
