@@ -2301,13 +2301,16 @@ __global__ void k_wrap_x(Grid g, float *a, float *b)
 // sampling run as separate launches; the per-cell arithmetic of a slot is
 // that of the one-thread-per-cell kernels.
 
-// FD order 12 with one slot per thread is held to 64 registers, so that 8 waves
-// fit a SIMD: the frame fetch had taken it to 66, and six EL_ISO shots of 1008 x
-// 707 with a damping frame from 61.9 to 63.2 us per step (61.9 again; with CPML
-// 66.6 and 65.8).  The other kernels of one slot per thread need 56 or fewer.
-template <int ND, int S>
-__global__ __launch_bounds__(BX *BY, ND == 6 && S == 1 ? 8 : 1) void k_velocity_b(Grid g, Fields f0, Mat m, int nt, const int *ntb, int fwi_acc)
+// PML: CPML frame.  One kernel for grids with and without needs 66 registers at
+// FD order 12 and one slot per thread, past the line for 8 waves per SIMD, and
+// more scalar registers at every order (EL_ISO with a damping frame, us per step
+// with that kernel and with its own: six shots of 1008 x 707 FD12 63.2 and 61.4,
+// FD8 51.8 and 49.7, two of 270 x 409 FD12 9.92 and 9.63).  Held to 64 registers
+// instead, it was 2 % slower on two small shots.
+template <int ND, int S, bool PML>
+__global__ __launch_bounds__(BX *BY) void k_velocity_b(Grid g, Fields f0, Mat m, int nt, const int *ntb, int fwi_acc)
 {
+    __builtin_assume(PML == (g.abs_type == 1));
     Park(*const park)[S] = reinterpret_cast<Park(*)[S]>(parks());
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
     const int2 t = tile_of(g, 0, 0, blockIdx.x);
@@ -4113,11 +4116,11 @@ void launch_blocks(sofi_dev *h, Grid gg, int lo, int hi, int S, A &&...a)
         launch_lds(h, K<1>::fn(), dim3(ntile, hi - r0), blk, park_bytes(gg, 1), gg, a...);
     }
 }
-template <int ND>
+template <int ND, bool PML>
 struct VelB {
     template <int S>
     struct K {
-        static auto fn() { return k_velocity_b<ND, S>; }
+        static auto fn() { return k_velocity_b<ND, S, PML>; }
     };
 };
 template <int ND, int WEQ>
@@ -4344,7 +4347,8 @@ int step_nd(sofi_dev *h, int nt, const int *ntb)
         }
         if (bm) {
             const int S = h->bs;
-            launch_blocks<ND, VelB<ND>::template K>(h, gg, lo, gg.k_hi, S, f, m, nt, ntb, fv.fwi_acc);
+            if (g.abs_type == 1) launch_blocks<ND, VelB<ND, true>::template K>(h, gg, lo, gg.k_hi, S, f, m, nt, ntb, fv.fwi_acc);
+            else launch_blocks<ND, VelB<ND, false>::template K>(h, gg, lo, gg.k_hi, S, f, m, nt, ntb, fv.fwi_acc);
             wrap_x(h, gg, lo, gg.k_hi, f.vx, f.vy);
             if (te && lo == lo0 && grp == span) {
                 (void)hipEventRecord(te[1], st);
