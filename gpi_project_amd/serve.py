@@ -21,10 +21,10 @@ device (one stream per handle).  Latency is completion time minus arrival
 time.  A request's results are those of the same request run alone: handles
 share nothing but the GPU, and a block boundary does not change a step.
 
-With worklist=True, small requests (one shot, at most lane_cells cells, a
-rheology whose update kernels run one thread per cell by default: VEL_ISO,
-VEL_VTI, AC_ISO) are admitted by footprint alone into a lane per FD order and
-rheology instead of a GPU worker.  A lane advances all its requests in blocks
+With worklist=True, small requests (one shot, at most lane_cells cells,
+VEL_ISO, VEL_VTI or AC_ISO) are admitted by footprint alone into a lane per FD
+order and rheology instead of a GPU worker.  EL_ISO and EL_VTI requests run on
+workers: lanes of theirs have not been measured.  A lane advances all its requests in blocks
 of lane_steps steps with sofi_run_many: each step's velocity and stress
 updates of all of them are one launch over a (handle, tile) work-list.
 Requests join a lane at the next block boundary and leave it when done, so
@@ -163,7 +163,7 @@ class Server:
             return None
         d = state.desc
         if (state.nshots != 1 or d.mode != 1 or d.fdorder_time != 2 or d.nx * d.ny > self.lane_cells
-                or d.weq not in (0, 3, 5)):          # AC_ISO, VEL_ISO, VEL_VTI (one thread per cell by default)
+                or d.weq not in (0, 3, 5)):          # AC_ISO, VEL_ISO, VEL_VTI
             return None
         return (d.fdorder, d.weq)
 

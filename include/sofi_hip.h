@@ -152,9 +152,11 @@ int sofi_run(sofi_dev *h, int nt_first, int nt_last);
  * block per item), waves (2, 4 or 8)} fixes the launch; NULL lets the first
  * call of a rheology, FD order, handle count and size measure waves 2, 4, 8
  * x rows 1, 2, 4 x blocks 0, 2048 on two steps each (after one untimed step;
- * the steps are part of the run) and keep the fastest in the process.  Each handle's results equal those of sofi_run with its update
- * kernels set to one thread per cell (sofi_set_launch), bit for bit, for any
- * launch, and the handle can go on with sofi_run afterwards.  The work runs
+ * the steps are part of the run) and keep the fastest in the process.  Each
+ * handle's results equal those of its own sofi_run bit for bit, for any
+ * launch, where its launch shapes are automatic or one thread per cell
+ * (sofi_set_launch; with a vector shape set: those of one thread per cell),
+ * and the handle can go on with sofi_run afterwards.  The work runs
  * on the first handle's stream; the call waits for it and sets every
  * handle's sofi_last_run_ms to the whole run's time (sofi_set_kernel_timing
  * does not sample its steps).  No counterpart in the reference, which runs
@@ -274,9 +276,11 @@ int sofi_fwi_residual_noalloc(sofi_dev *h, const sofi_residual_opts *opts, const
  * two / four consecutive cells of a row (vector loads and stores) in
  * 128 x 4 / 256 x 4 tiles, SOFI_LAUNCH_AUTO (the default) the shape
  * measured fastest (CELL, for EL_ISO with VEC2's rounding of the stress
- * update), for one-shot handles and batches alike.  Results agree to
- * rounding between shapes and bit for bit between a batch slot and a
- * one-shot handle of the same shape. */
+ * update), for one-shot handles and a batch's slot loops alike.  Results
+ * agree to rounding between shapes and bit for bit between a slot of a slot
+ * loop and a one-shot handle of the same shape (VEL_VTI: to rounding).  Slot
+ * blocks (sofi_set_batch_block) take no shape: theirs is one thread per cell,
+ * with CELL's rounding for EL_ISO. */
 enum { SOFI_LAUNCH_AUTO = 0, SOFI_LAUNCH_CELL = 1, SOFI_LAUNCH_VEC2 = 2, SOFI_LAUNCH_VEC4 = 3 };
 int sofi_set_launch(sofi_dev *h, int velocity_shape, int stress_shape);
 
