@@ -3132,6 +3132,15 @@ bool one_launch_fits(const sofi_desc &d, int nshots)
            d.seismo != 3 && d.seismo != 4 && (size_t)d.nx * d.ny <= ONE_LAUNCH_CELLS;
 }
 
+// Floats of the second set's arrays, each on a 256-B line: five planes, two
+// x-frame and two y-frame CPML arrays
+struct NextSize {
+    size_t plane, x, y;
+    NextSize(size_t pl, size_t nxp, size_t nyp)
+        : plane((pl + 63) / 64 * 64), x((nxp + 63) / 64 * 64), y((nyp + 63) / 64 * 64) {}
+    size_t all() const { return 5 * plane + 2 * x + 2 * y; }
+};
+
 int dalloc(sofi_dev *h, void **p, size_t bytes)
 {
     if (bytes == 0) bytes = 4;
@@ -3398,11 +3407,21 @@ int sofi_open_batch(const sofi_desc *desc, int nshots, sofi_dev **out)
         rc |= dalloc_t(h, &f.psi_vxy, nyp);
     }
     if (one_launch_fits(d, nshots)) {
+        // one allocation: nine would make opening a small grid a fifth longer
+        const NextSize z(pl, f.psi_sxx_x ? (size_t)g.nxp : 0, f.psi_sxx_x ? (size_t)g.nyp : 0);
         Next &n = h->alt;
-        for (float **q : { &n.vx, &n.vy, &n.sxx, &n.syy, &n.sxy }) rc |= dalloc_t(h, q, pl);
-        if (f.psi_sxx_x) {
-            for (float **q : { &n.psi_sxx_x, &n.psi_sxy_x }) rc |= dalloc_t(h, q, (size_t)g.nxp);
-            for (float **q : { &n.psi_syy_y, &n.psi_sxy_y }) rc |= dalloc_t(h, q, (size_t)g.nyp);
+        rc |= dalloc_t(h, &n.vx, z.all());
+        if (!rc) {
+            n.vy = n.vx + z.plane;
+            n.sxx = n.vy + z.plane;
+            n.syy = n.sxx + z.plane;
+            n.sxy = n.syy + z.plane;
+        }
+        if (!rc && f.psi_sxx_x) {
+            n.psi_sxx_x = n.sxy + z.plane;
+            n.psi_sxy_x = n.psi_sxx_x + z.x;
+            n.psi_syy_y = n.psi_sxy_x + z.x;
+            n.psi_sxy_y = n.psi_syy_y + z.y;
         }
     }
     if (d.mode == SOFI_MODE_FWI) {
@@ -5709,8 +5728,8 @@ size_t sofi_estimate_footprint(const sofi_desc *d, int nshots, int ntr, int nsna
     const size_t mx = (size_t)(d->ny + 1) * wx * 4 * nb + A, my = wx * (size_t)(d->nx + 1) * 4 * nb + A;
     const bool cpml = d->abs_type == 1 && d->fw > 0, second = one_launch_fits(*d, nshots);
     if (cpml) b += 4 * mx + 4 * my;
-    if (second) b += 5 * (pl + A);
-    if (second && cpml) b += 2 * mx + 2 * my;
+    if (second)
+        b += NextSize(pl / 4, cpml ? (size_t)(d->ny + 1) * wx : 0, cpml ? wx * (size_t)(d->nx + 1) : 0).all() * 4 + A;
     size_t arrays = 4;                                                        // rip rjp pu ppi
     switch (d->weq) {
       case SOFI_EL_ISO: arrays += 3; break;
