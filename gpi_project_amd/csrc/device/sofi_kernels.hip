@@ -3935,8 +3935,8 @@ int vec_width(int shape)
     // fastest shape at nearly every size (GLUPS, CELL / VEC2 / VEC4: EL_ISO FD8
     // 1500 x 500 41.2 / 34.2 / 35.9, 2000 x 1000 60.0 / 51.8 / 55.9, 2741 x 1313
     // 66.3 / 61.1 / 61.8, 4000 x 2000 67.5 / 47.0 / 56.9; EL_VTI FD6 2000 x 1000
-    // 59.5 / 59.0 / 58.9, 3000 x 1700 70.1 / 75.8 / 69.1, 4000 x 2000 68.8 / 52.5
-    // / 61.4; VEL_ISO L = 3 FD8 1000 x 1000 30.1 / 28.5 / 25.9, 2000 x 1000 37.4 /
+    // 59.5 / 59.0 / 58.9, 3000 x 1700 70.1 / 75.8 / 69.1 in plain order and CELL 87.0
+    // in bands, 4000 x 2000 68.8 / 52.5 / 61.4; VEL_ISO L = 3 FD8 1000 x 1000 30.1 / 28.5 / 25.9, 2000 x 1000 37.4 /
     // 36.2 / 35.8, 4000 x 2000 37.5 / 27.1 / 28.8)
     return 1;
 }
